@@ -38,8 +38,17 @@ using namespace opsmi;
 
 namespace {
 
-constexpr int kRows2D = 4;  // rows per wave of a 2D tile (tile = 64 x 16)
-constexpr int kChunk3D = 16;
+// Default tile parameter per size class (size_class): rows per wave of a 2D
+// tile, z planes of a 3D tile.  A tile is worked through serially, so small
+// solves take short tiles (more workgroups) and large ones long tiles (fewer
+// rim re-reads).  Microseconds per CG iteration of one solve alone:
+//   2D side    1 row   2 rows  4 rows   |  3D side   4      8      16 planes
+//     256       17.9    18.6    20.2    |    32     23.5   30.0   42.3
+//     512       20.1    19.6    21.0    |    64     24.7   29.8   41.0
+//    1000       35.7    29.4    28.0    |    96     42.4   41.2   51.4
+//    2000      104.9    85.6    76.5    |   200    242.4  261.1  197.5
+constexpr int kRows2D[3] = {1, 2, 4};
+constexpr int kChunk3D[3] = {4, 4, 16};
 constexpr int kPart = 4;  // partial sums per tile (stride of the partials array)
 
 struct SolveDev {
@@ -216,6 +225,16 @@ __device__ __forceinline__ T op5(const Row5<T, V> &R, int j, int n) {
   return (T)4.0 * R.c[j] - (xm + xp) - (R.up[j] + R.dn[j]);
 }
 
+// First tile of this workgroup.  XCD k takes the k-th contiguous eighth of
+// the tiles in flight: of the whole grid's when the table is longer than the
+// grid, otherwise of the table's.  (Numbered over the grid, a table of 504
+// tiles filled 2 of the 8 XCDs: a 1000^2 Poisson iteration took 64.9 us,
+// spread over all eight 28.0; a 128^3 heat iteration 222.6 and 60.8.)
+__device__ __forceinline__ int first_tile(int nt) {
+  const int nb = min(nt, (int)gridDim.x);
+  return (int)blockIdx.x < nb ? (int)xcd_tile(blockIdx.x, (unsigned)nb) : nt;
+}
+
 // ------------------------------------------------------------ iteration
 __global__ __launch_bounds__(256) void sk_calc_w(const SolveDev *S, const SolveStat *st, const int2 *tiles,
                                                  const int *ntiles, double *part) {
@@ -223,7 +242,7 @@ __global__ __launch_bounds__(256) void sk_calc_w(const SolveDev *S, const SolveS
   __shared__ double sh[16][1];
   __shared__ double sh3[16][3];
   const int nt = *ntiles;
-  for (int t = (int)xcd_tile(blockIdx.x, gridDim.x); t < nt; t += (int)gridDim.x) {
+  for (int t = first_tile(nt); t < nt; t += (int)gridDim.x) {
     const int2 e = tiles[t];
     if (st[e.x].done) continue;
     const SolveDev d = S[e.x];
@@ -322,7 +341,7 @@ __global__ __launch_bounds__(256) void sk_update(const SolveDev *S, const SolveS
   __shared__ double sh[16][1];
   __shared__ double sh3[16][3];
   const int nt = *ntiles;
-  for (int t = (int)xcd_tile(blockIdx.x, gridDim.x); t < nt; t += (int)gridDim.x) {
+  for (int t = first_tile(nt); t < nt; t += (int)gridDim.x) {
     const int2 e = tiles[t];
     if (st[e.x].done) continue;
     const SolveDev d = S[e.x];
@@ -425,7 +444,7 @@ __global__ __launch_bounds__(256) void sk_update(const SolveDev *S, const SolveS
 __global__ __launch_bounds__(256) void sk_axpby(const SolveDev *S, const SolveStat *st, const int2 *tiles,
                                                 const int *ntiles) {
   const int nt = *ntiles;
-  for (int t = (int)xcd_tile(blockIdx.x, gridDim.x); t < nt; t += (int)gridDim.x) {
+  for (int t = first_tile(nt); t < nt; t += (int)gridDim.x) {
     const int2 e = tiles[t];
     if (st[e.x].done) continue;
     const SolveDev d = S[e.x];
@@ -805,10 +824,10 @@ struct opsmi_server_s {
   int next_id = 0, n_active = 0;
   long tiles_active = 0;  // tiles of the admitted solves (the next table)
   // tile parameter per size class (defaults; opsmi_serve_autotune measures)
-  int chunk3d[3] = {kChunk3D, kChunk3D, kChunk3D};
-  int chunk3d_mixed[3] = {kChunk3D, kChunk3D, kChunk3D};  // FP32-inner heat solves
-  int rows2d[3] = {kRows2D, kRows2D, kRows2D};
-  int rows2d_mixed[3] = {kRows2D, kRows2D, kRows2D};  // FP32-inner solves
+  int chunk3d[3] = {kChunk3D[0], kChunk3D[1], kChunk3D[2]};
+  int chunk3d_mixed[3] = {kChunk3D[0], kChunk3D[1], kChunk3D[2]};  // FP32-inner heat solves
+  int rows2d[3] = {kRows2D[0], kRows2D[1], kRows2D[2]};
+  int rows2d_mixed[3] = {kRows2D[0], kRows2D[1], kRows2D[2]};  // FP32-inner solves
 };
 
 namespace {
@@ -1062,8 +1081,10 @@ opsmi_server opsmi_serve_create(size_t hbm_budget, int max_slots, int iters_per_
   if (const char *e = getenv("OPSMI_SERVE_GRAPH"))
     if (e[0] == '0') S->use_graph = 0;
   S->grid = inst().num_cus * 8;
-  // smallest tile: a 2D tile of 64 x 8 points (2 rows per wave) over 4 fields
-  S->max_tiles = std::min<size_t>(S->budget / (size_t)(kWave * kWavesPerBlock * 2 * 4 * 8) + (size_t)max_slots * 8,
+  // the least memory a tile stands for: 128 x 4 points (one row per wave)
+  // over 4 fields, half of it used in the worst row (129 points in rows of
+  // 160); solves of fewer points than that have at most 8 tiles
+  S->max_tiles = std::min<size_t>(S->budget / 8192 + (size_t)max_slots * 8,
                                   (size_t)1 << 25);
   OPSMI_HIP(hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking));
   OPSMI_HIP(hipMalloc(&S->arena_base, S->budget));
@@ -1072,7 +1093,7 @@ opsmi_server opsmi_serve_create(size_t hbm_budget, int max_slots, int iters_per_
   OPSMI_HIP(hipMalloc(&S->d_stat, sizeof(SolveStat) * max_slots));
   OPSMI_HIP(hipMalloc(&S->d_tiles, sizeof(int2) * S->max_tiles));
   OPSMI_HIP(hipMalloc(&S->d_ntiles, sizeof(int)));
-  OPSMI_HIP(hipMalloc(&S->d_part, sizeof(double) * S->max_tiles));
+  OPSMI_HIP(hipMalloc(&S->d_part, sizeof(double) * kPart * S->max_tiles));
   OPSMI_HIP(hipMalloc(&S->d_setup_part, sizeof(double) * S->max_tiles));
   OPSMI_HIP(hipHostMalloc((void **)&S->h_stat, sizeof(SolveStat) * max_slots, hipHostMallocDefault));
   OPSMI_HIP(hipMemsetAsync(S->d_stat, 0, sizeof(SolveStat) * max_slots, S->stream));

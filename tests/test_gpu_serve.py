@@ -248,3 +248,18 @@ def test_request_stream_driver(gpu_ops):
     for k, n, s, it in zip(kinds, sizes, seeds, iters):
         d, _ = _run_alone(S, k, n, s)
         assert d["iters"] == it
+
+
+@pytest.mark.parametrize("n", [3, 5, 33, 255, 257, 1023, 1024, 2048, 2300])
+def test_tile_tables_from_one_tile_to_more_than_the_grid(serve, n):
+    # 1, 2, 9, 2 x 64, 3 x 33, 8 x 128, 8 x 64, 16 x 128 (the grid) and 18 x 144
+    # tiles: each is worked on once an iteration.  Four CG iterations against
+    # the oracle's: sums of n^2 terms in another order, 1e-12.
+    S = serve
+    srv = S.Server(budget_bytes=1 << 28, max_slots=2)
+    i = srv.submit(S.POISSON2D, n, seed=SEED, max_iters=4)
+    done, x = srv.run()[i]
+    srv.close()
+    ref = O.poisson_cg(2, n, n, 1, O.poisson_rhs(SEED, 2, n, n), max_iters=4, tol=1e-10, nthreads=8)
+    assert done["iters"] == ref["iters"]
+    assert np.max(np.abs(x - ref["x"])) <= 1e-12 * np.max(np.abs(ref["x"]))
