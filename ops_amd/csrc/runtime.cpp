@@ -1,6 +1,7 @@
 // Host runtime of the MI355X OPS backend: lifecycle, declarations, arguments,
 // HBM-resident dats with lazy host mirrors, reductions, statistics and the
 // C ABI wrappers for all of them.
+#include "box.h"
 #include "runtime.h"
 
 #include <float.h>
@@ -100,6 +101,16 @@ DatView view_of(ops_dat d) {
 static DatImpl *impl(ops_dat d) { return (DatImpl *)d->impl; }
 
 static size_t dat_lead(ops_dat d) { return (size_t)(d->data_d - impl(d)->alloc); }
+
+// whether a caller's buffer is device memory (fetch and set take either kind)
+bool device_pointer(const void *p) {
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();  // memory that HIP does not know: the host's
+    return false;
+  }
+  return at.type == hipMemoryTypeDevice;
+}
 
 void ensure_host(ops_dat d) {
   Instance &I = inst();
@@ -838,6 +849,7 @@ void ops_exit(void) {
   (void)hipFree(I.d_partials2);
   I.d_partials2 = nullptr;
   (void)hipHostFree(I.h_pinned);
+  I.staging.release();
   (void)hipHostFree(I.h_hfold);
   I.h_hfold = nullptr;
   I.d_hfold = nullptr;
@@ -957,10 +969,19 @@ ops_dat ops_decl_dat_char(ops_block block, int dim, int *dsize, int *base, int *
     size_t rows = 1;
     for (int n = 1; n < nd; n++) rows *= d->size[n];
     const int ncomp = m->soa ? dim : 1;
-    for (int c = 0; c < ncomp; c++)
-      OPSMI_HIP(hipMemcpy2D(d->data_d + (size_t)c * row * rows + (size_t)c * d->x_pad * unit * rows,
-                            row + (size_t)d->x_pad * unit, data + (size_t)c * upitch * rows, upitch, upitch, rows,
-                            hipMemcpyHostToDevice));
+    const bool on_device = device_pointer(data);
+    for (int c = 0; c < ncomp; c++) {
+      Box b;
+      b.pitch = (long)(row + (size_t)d->x_pad * unit);
+      b.plane = b.pitch * d->size[1];
+      b.base = d->data_d + (size_t)c * b.pitch * rows;
+      b.width = upitch;
+      b.rows = (unsigned)d->size[1];
+      b.planes = (unsigned)(rows / d->size[1]);
+      char *from = data + (size_t)c * upitch * rows;
+      if (on_device) OPSMI_HIP(hipMemcpy2D(b.base, b.pitch, from, upitch, upitch, rows, hipMemcpyDefault));
+      else box_copy(I.staging, I.stream, b, from, true);
+    }
   }
   d->data = nullptr;
   d->user_managed = 0;
@@ -1380,7 +1401,7 @@ void ops_dat_release_raw_data_memspace(ops_dat dat, int part, ops_access acc, op
 }
 
 // copies a box [lo,hi) of points between the dat's device array and a dense
-// buffer (x fastest), one 2D copy per z-plane
+// buffer (x fastest, a point's components together, in either layout)
 static void slab_copy(ops_dat dat, char *buf, const int *lo, const int *hi, bool to_dat) {
   Instance &I = inst();
   int nd = dat->block->dims;
@@ -1392,43 +1413,34 @@ static void slab_copy(ops_dat dat, char *buf, const int *lo, const int *hi, bool
     if (l[d] < first || h[d] > last || h[d] < l[d])
       fail(OPS_INVALID_ARGUMENT, cat("slab [", l[d], ",", h[d], ") outside dat ", dat->name, " in dimension ", d));
   }
-  size_t es = dat->elem_size;
-  size_t w = (size_t)(h[0] - l[0]) * es, rows = (size_t)(h[1] - l[1]);
+  const size_t es = dat->elem_size, ts = dat->type_size;
+  const size_t w = (size_t)(h[0] - l[0]) * es, rows = (size_t)(h[1] - l[1]);
   if (w == 0 || rows == 0 || h[2] <= l[2]) return;
-  DatView v = view_of(dat);
-  size_t pitch = (size_t)v.sy * dat->type_size;
-  if (impl(dat)->soa) {
-    // the buffer holds the points' components together, as the reference's
-    // slab copy presents a SoA dat (ops/c/src/externlib/ops_util.cpp:353-500):
-    // each component's box goes through a component-major staging copy
-    const size_t ts = dat->type_size, nc = dat->dim;
-    const size_t wx = (size_t)(h[0] - l[0]), planes = (size_t)(h[2] - l[2]), np = wx * rows * planes;
-    std::vector<char> tmp(np * es);
-    if (to_dat)
-      for (size_t p = 0; p < np; p++)
-        for (size_t c = 0; c < nc; c++) memcpy(&tmp[(c * np + p) * ts], buf + (p * nc + c) * ts, ts);
-    for (size_t c = 0; c < nc; c++)
-      for (int z = l[2]; z < h[2]; z++) {
-        char *dp = v.base + ((long)c * v.cs + (long)l[0] + (long)l[1] * v.sy + (long)z * v.sz) * (long)ts;
-        char *bp = &tmp[(c * np + (size_t)(z - l[2]) * wx * rows) * ts];
-        if (to_dat)
-          OPSMI_HIP(hipMemcpy2DAsync(dp, pitch, bp, wx * ts, wx * ts, rows, hipMemcpyDefault, I.stream));
-        else
-          OPSMI_HIP(hipMemcpy2DAsync(bp, wx * ts, dp, pitch, wx * ts, rows, hipMemcpyDefault, I.stream));
-      }
+  const DatView v = view_of(dat);
+  const bool soa = impl(dat)->soa;
+  Box b;
+  b.base = v.base + ((long)l[0] * v.sx + (long)l[1] * v.sy + (long)l[2] * v.sz) * (long)ts;
+  b.pitch = v.sy * (long)ts;
+  b.plane = v.sz * (long)ts;
+  b.width = w;
+  b.rows = (unsigned)rows;
+  b.planes = (unsigned)(h[2] - l[2]);
+  if (soa) {
+    b.comps = (unsigned)dat->dim;
+    b.elem = (unsigned)ts;
+    b.cstride = v.cs * (long)ts;
+  }
+  if (!device_pointer(buf)) {
+    box_copy(I.staging, I.stream, b, buf, to_dat);
     OPSMI_HIP(hipStreamSynchronize(I.stream));
-    if (!to_dat)
-      for (size_t p = 0; p < np; p++)
-        for (size_t c = 0; c < nc; c++) memcpy(buf + (p * nc + c) * ts, &tmp[(c * np + p) * ts], ts);
     return;
   }
-  for (int z = l[2]; z < h[2]; z++) {
-    char *dp = v.base + ((long)l[0] * dat->dim + (long)l[1] * v.sy + (long)z * v.sz) * dat->type_size;
-    char *bp = buf + (size_t)(z - l[2]) * w * rows;
-    if (to_dat)
-      OPSMI_HIP(hipMemcpy2DAsync(dp, pitch, bp, w, w, rows, hipMemcpyDefault, I.stream));
-    else
-      OPSMI_HIP(hipMemcpy2DAsync(bp, w, dp, pitch, w, rows, hipMemcpyDefault, I.stream));
+  if (soa)
+    fail(OPS_NOT_IMPLEMENTED, cat("dat ", dat->name, ": a structure-of-arrays dat is copied from and to host memory only"));
+  for (unsigned z = 0; z < b.planes; z++) {
+    char *dp = b.base + (long)z * b.plane, *bp = buf + (size_t)z * w * rows;
+    if (to_dat) OPSMI_HIP(hipMemcpy2DAsync(dp, b.pitch, bp, w, w, rows, hipMemcpyDefault, I.stream));
+    else OPSMI_HIP(hipMemcpy2DAsync(bp, w, dp, b.pitch, w, rows, hipMemcpyDefault, I.stream));
   }
   OPSMI_HIP(hipStreamSynchronize(I.stream));
 }

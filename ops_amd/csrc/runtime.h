@@ -111,6 +111,15 @@ struct Const {
   std::vector<char> bytes;
 };
 
+// Pinned buffers of one owner (the library, a server): used by one call at a
+// time, idle when box_copy returns.
+struct Staging {
+  char *host[2] = {}, *dev[2] = {};
+  hipEvent_t ev[2] = {};
+  void ensure();
+  void release();
+};
+
 struct Instance {
   bool initialised = false;
   int diags = 1;
@@ -151,6 +160,9 @@ struct Instance {
 
   // host staging for reduction results
   void *h_pinned = nullptr;
+
+  // pinned buffers of fetches, sets and declarations with data
+  Staging staging;
 
   // Host fold of a result read right away: the one loop of a flush that
   // reduces into the handle being read (FP64, first use since the last

@@ -31,6 +31,7 @@
 
 #include "../../include/ops_mi355x_serve.h"
 #include "../apps/problems.h"
+#include "box.h"
 #include "engine.h"
 #include "column.h"
 
@@ -813,6 +814,7 @@ struct opsmi_server_s {
   int *d_ntiles = nullptr;
   double *d_part = nullptr, *d_setup_part = nullptr;
   SolveStat *h_stat = nullptr;  // pinned
+  Staging staging;              // fetched solutions
   std::vector<SolveDev> h_solves;
   std::vector<int> slot_req;
   std::vector<int2> h_tiles;
@@ -1188,10 +1190,21 @@ int opsmi_serve_fetch(opsmi_server S, int id, double *out) {
   Req &R = find(S, id);
   if (R.state != 2) fail(OPS_INVALID_ARGUMENT, cat("opsmi_serve_fetch: solve ", id, " has not completed"));
   const SolveDev &d = R.dev;
-  for (int z = 0; z < d.nz; z++)
-    OPSMI_HIP(hipMemcpy2DAsync(out + (size_t)z * d.nx * d.ny, (size_t)d.nx * 8, d.u + (long)z * d.sz,
-                               (size_t)d.sy * 8, (size_t)d.nx * 8, (size_t)d.ny, hipMemcpyDeviceToHost, S->stream));
-  OPSMI_HIP(hipStreamSynchronize(S->stream));
+  Box b;
+  b.base = (char *)d.u;
+  b.pitch = d.sy * 8;
+  b.plane = d.sz * 8;
+  b.width = (size_t)d.nx * 8;
+  b.rows = (unsigned)d.ny;
+  b.planes = (unsigned)d.nz;
+  if (device_pointer(out)) {
+    for (int z = 0; z < d.nz; z++)
+      OPSMI_HIP(hipMemcpy2DAsync(out + (size_t)z * d.nx * d.ny, b.width, d.u + (long)z * d.sz, b.pitch, b.width,
+                                 (size_t)d.ny, hipMemcpyDeviceToDevice, S->stream));
+    OPSMI_HIP(hipStreamSynchronize(S->stream));
+  } else {
+    box_copy(S->staging, S->stream, b, (char *)out, false);
+  }
   free_req(S, id);
   return 0;
   OPSMI_API_END(-1)
@@ -1303,6 +1316,7 @@ void opsmi_serve_destroy(opsmi_server S) {
   (void)hipFree(S->d_part);
   (void)hipFree(S->d_setup_part);
   (void)hipHostFree(S->h_stat);
+  S->staging.release();
   if (S->stream) (void)hipStreamDestroy(S->stream);
   delete S;
 }

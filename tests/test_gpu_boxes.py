@@ -1,0 +1,66 @@
+"""Boxes of points between dats and host arrays (fetch, set, slabs,
+declarations with data): bytes, so equal to numpy's slices exactly.  Sizes
+around the copy's pieces (4 MiB) and units (1 to 16 bytes)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # size (x first), halo, components, structure of arrays, type
+    ([524288], 1, 1, False, np.float64),         # one row: a piece and two halo points
+    ([3], 1, 1, False, np.float32),
+    ([1031, 700], 2, 1, False, np.float64),      # odd rows, two pieces
+    ([1500, 1400], 1, 1, False, np.float32),     # three pieces, 16-byte units inside a row
+    ([33, 17, 9], 1, 1, False, np.float64),
+    ([130, 64, 70], 3, 1, False, np.float32),
+    ([37, 20, 11], 1, 3, False, np.float64),
+    ([37, 20, 11], 1, 3, True, np.float64),
+    ([600, 300, 9], 1, 3, True, np.float32),     # components together, two pieces
+    ([257, 190], 1, 2, True, np.int32),
+]
+
+
+@pytest.mark.parametrize("size,halo,dim,soa,dtype", CASES)
+def test_boxes_equal_numpy_slices(gpu_ops, size, halo, dim, soa, dtype):
+    ops = gpu_ops
+    nd = len(size)
+    ops.ops_set_soa(soa)
+    try:
+        blk = ops.ops_decl_block(nd, "boxes")
+        d = ops.ops_decl_dat(blk, size, [-halo] * nd, [halo] * nd, dtype, "d", dim=dim)
+    finally:
+        ops.ops_set_soa(False)
+    # the dat's x padding belongs to its upper halo (d_p as declared here)
+    shape = tuple(n + 2 * halo for n in reversed(size)) + ((dim,) if dim > 1 else ())
+    rng = np.random.RandomState(7)
+    ref = (rng.randint(-2 ** 30, 2 ** 30, shape)).astype(dtype)
+    ops.set_whole(d, ref)
+    assert np.array_equal(ops.get_whole(d), ref)
+    inner = tuple(slice(halo, -halo) for _ in size)
+    if dim == 1:
+        assert np.array_equal(ops.ops_dat_fetch_data(d), ref[inner])
+        new = (rng.randint(-2 ** 30, 2 ** 30, ref[inner].shape)).astype(dtype)
+        ops.ops_dat_set_data(d, new)
+        ref[inner] = new
+        assert np.array_equal(ops.get_whole(d), ref)
+    # a slab off every alignment: [1, n - 1) in each dimension
+    slab = [v for n in size for v in (1, n - 1)]
+    at = tuple(slice(halo + 1, halo + n - 1) for n in reversed(size))
+    assert np.array_equal(ops.ops_dat_fetch_data_slab(d, slab), ref[at])
+    new = (rng.randint(-2 ** 30, 2 ** 30, ref[at].shape)).astype(dtype)
+    ops.ops_dat_set_data_slab(d, slab, new)
+    ref[at] = new
+    assert np.array_equal(ops.get_whole(d), ref)
+    ops.ops_free_dat(d)
+
+
+@pytest.mark.parametrize("size", [[5], [700, 300], [1031, 700], [40, 30, 20]])
+def test_declaration_with_data(gpu_ops, size):
+    ops = gpu_ops
+    nd = len(size)
+    shape = tuple(n + 2 for n in reversed(size))
+    data = np.random.RandomState(3).rand(*shape)
+    d = ops.ops_decl_dat(ops.ops_decl_block(nd, "withdata"), size, data=data, name="d")
+    assert np.array_equal(ops.get_whole(d), data)
+    ops.ops_free_dat(d)
