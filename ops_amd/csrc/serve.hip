@@ -4,20 +4,24 @@
 // Device side.  Each active solve (one block) is described by a SolveDev
 // (field pointers, strides, sizes, tile grid) and a SolveStat (CG scalars
 // and status) in device memory.  A tile table lists (solve, tile) pairs of
-// every active solve, contiguous per solve.  One CG iteration is five
+// every active solve, contiguous per solve.  One CG iteration is two
 // launches, each persistent (a fixed grid walks the tile table; blocks are
 // renumbered so each XCD walks a contiguous stretch of tiles):
-//   sk_calc_w    w = A p per tile, partial p.w per tile
-//   sk_fold<0>   per solve: pw = fold of its partials, alpha = rro / pw
-//   sk_update    u += alpha p ; r -= alpha w, partial r.r per tile
-//   sk_fold<1>   per solve: rrn, beta = rrn / rro, rro = rrn, stop test
-//   sk_axpby     p = beta p + r
+//   sk_sweep     rrn = fold of r.r ; beta = rrn / rro, stop test ;
+//                w = A (beta p + r) per tile, partial p.w per tile
+//   sk_update    pw = fold of p.w ; alpha = rro / pw ;
+//                p = beta p + r ; u += alpha p ; r -= alpha w, partial r.r
+// Every workgroup folds its solve's partials itself, in the same fixed order,
+// so no launch waits for a fold of its own; the sweep forms the new p at the
+// points its stencil reads and the update, pointwise, stores it.  (Five
+// launches, with folds and p update of their own, took 17.5 us an iteration
+// on a small solve.)  The CG scalars alternate between two copies: a launch
+// reads one, and its solve's first tile writes the other.  sk_finish folds
+// the last r.r of a batch of iterations and tests it.
 // Solves that are done skip all work, so a graph of K iterations stops each
-// solve exactly where it converges.  Partials are folded per solve, in a
-// fixed order, by one workgroup: a solve's numbers do not depend on the rest
-// of the batch.  3D heat tiles are 128 x 4 x chunk z-marching columns
-// (heat3_column_v, two points per lane); 2D Poisson tiles are 128 x (4 chunk)
-// rows, two points per lane.
+// solve exactly where it converges.  A solve's numbers do not depend on the
+// rest of the batch.  3D heat tiles are 128 x 4 x chunk columns marched along
+// z in registers, 2D Poisson tiles 128 x (4 chunk) rows, two points per lane.
 //
 // Host side.  Fields live in one arena of the HBM budget (first-fit, 256 B
 // granules, coalescing).  A step admits queued solves in FIFO order while a
@@ -50,7 +54,7 @@ namespace {
 //    2000      104.9    85.6    76.5    |   200    242.4  261.1  197.5
 constexpr int kRows2D[3] = {1, 2, 4};
 constexpr int kChunk3D[3] = {4, 4, 16};
-constexpr int kPart = 4;  // partial sums per tile (stride of the partials array)
+constexpr int kPart = 4;  // partial sums per tile: planes 0-2 of the update, plane 3 p.w
 
 struct SolveDev {
   double *u, *p, *r, *w, *kx, *ky, *kz;  // element (0,0,0) of each field
@@ -74,11 +78,13 @@ struct SolveDev {
 
 // phases of a mixed solve: the next iteration runs an inner FP32 PCG step,
 // or applies the correction x += e and recomputes the FP64 residual
-enum { PH_INNER = 0, PH_RESID = 1 };
+// (3D heat: applies it in one iteration, PH_CORR, and recomputes in the next)
+enum { PH_INNER = 0, PH_RESID = 1, PH_CORR = 2 };
 
 struct SolveStat {
   double rro, rr0, stop, pw, alpha, beta;
-  int iters, done, max_iters, pad;
+  int iters, done, max_iters;
+  int pending;  // an update's sums are still to be folded
   // mixed: inner r.z, inner stop threshold, |f|, targets
   double rz, istop, fn, tol, inner_tol;
   int phase, outer, max_outer, axpby;  // axpby: the next p update runs
@@ -196,13 +202,6 @@ struct HeatOutResid {
   }
 };
 
-// LDS of the calc_w pass: the FP64 heat column (2 doubles per lane) or its
-// FP32 form (4 floats per lane); both are 31 KB
-union CalcWLds {
-  HeatLdsV<kSV, kWavesPerBlock> d;
-  HeatLdsV<kSV, kWavesPerBlock, float> f;
-};
-
 // the 2D 5-point operator over a group: the group's row and the rows above
 // and below, and the neighbours just left and right of the group
 template <class T, int V>
@@ -237,159 +236,556 @@ __device__ __forceinline__ int first_tile(int nt) {
 }
 
 // ------------------------------------------------------------ iteration
-__global__ __launch_bounds__(256) void sk_calc_w(const SolveDev *S, const SolveStat *st, const int2 *tiles,
-                                                 const int *ntiles, double *part) {
-  __shared__ CalcWLds lds;
-  __shared__ double sh[16][1];
-  __shared__ double sh3[16][3];
-  const int nt = *ntiles;
-  for (int t = first_tile(nt); t < nt; t += (int)gridDim.x) {
-    const int2 e = tiles[t];
-    if (st[e.x].done) continue;
-    const SolveDev d = S[e.x];
-    const TileBox b = tile_box(d, e.y);
-    double acc = 0.0;
-    if (d.mixed && d.kind == OPSMI_SOLVE_HEAT3D) {
-      __syncthreads();  // LDS of the previous tile fully read
-      if (st[e.x].phase == PH_RESID) {
-        // FP64 residual of the corrected x (the correction x += e ran in the
-        // previous iteration's last pass) and the inner start
-        const Ptr<const double> f = PC(d.f, d);
-        const Ptr<float> rr = PF32(d.r32, d), ev = PF32(d.e32, d), p = PF32(d.p32, d);
-        // (the FP64 column covers 64 kSV points; a wider tile in parts)
-        HeatOutResid out{f, rr, ev, p};
-        for (int h = 0; h < d.sv / kSV; h++) {
-          const int x0 = b.x0 + h * kWave * kSV;
-          if (x0 >= d.nx) break;  // (uniform over the workgroup)
-          if (h > 0) __syncthreads();  // LDS of the previous half fully read
-          heat3_column_out<double, kSV, kWavesPerBlock, 1>(lds.d, out, PC(d.kx, d), PC(d.ky, d), PC(d.kz, d),
-                                                           PC(d.u, d), d.rx, d.ry, d.rz, x0, b.y0, d.nx, d.ny, b.z0,
-                                                           b.z1);
-        }
-        store_partials<3>(out.acc, part + (size_t)t * kPart, sh3);
-        continue;
-      }
-      // inner sweep in FP32 with float coefficients: w = A p, p.w in FP64
-      const Ptr<float> w = PF32(d.w32, d);
-      HeatOutW<float, kSV, false> out{w};
-      heat3_column_out<float, kSV, kWavesPerBlock, 1>(lds.f, out, PF32C(d.kx32, d), PF32C(d.ky32, d),
-                                                      PF32C(d.kz32, d), PF32C(d.p32, d), (float)d.rx, (float)d.ry,
-                                                      (float)d.rz, b.x0, b.y0, d.nx, d.ny, b.z0, b.z1);
-      store_partial(out.acc, part + (size_t)t * kPart, sh);
-      continue;
-    }
-    if (d.mixed) {
-      if (st[e.x].phase == PH_RESID) {
-        // the correction x = x + (double) e (pointwise; the residual follows
-        // in sk_update once every tile has applied it)
-        const Ptr<double> x = P(d.u, d);
-        const Ptr<const float> ev = PF32C(d.e32, d);
-        tile_groups<kSV32>(d, b, [&](int i, int j, int k, int n) {
-          double xv[kSV32];
-          float evv[kSV32];
-          ldv<double, kSV32>(x.at(i, j, k), n, xv);
-          ldv<float, kSV32>(ev.at(i, j, k), n, evv);
+// Sums of a solve's partials [tile0, tile0 + ntiles) of planes first ..
+// first + D - 1, in thread 0.  Thread i adds partials i, i + 256, ... in that
+// order; eight are loaded before they are added (eight loads in flight, the
+// same sums).
+template <int D>
+__device__ __forceinline__ void fold_partials(const double *part, size_t np, int first, int t0, int n,
+                                              double (&acc)[D], double (*sh)[D]) {
+  const int tid = (int)(threadIdx.x + threadIdx.y * blockDim.x);
 #pragma unroll
-          for (int q = 0; q < kSV32; q++) xv[q] = xv[q] + (double)evv[q];
-          stv<double, kSV32, false>(x.at(i, j, k), n, xv);
-        });
-        continue;
-      }
-      // inner sweep in FP32: w = 4p - (p(-1,0) + p(1,0)) - (p(0,-1) + p(0,1)), p.w in FP64
-      const Ptr<const float> p = PF32C(d.p32, d);
-      const Ptr<float> w = PF32(d.w32, d);
-      tile_groups<kSV32>(d, b, [&](int i, int j, int k, int n) {
-        Row5<float, kSV32> R;
-        load5<float, kSV32>(p, i, j, n, R);
-        float v[kSV32];
+  for (int k = 0; k < D; k++) acc[k] = 0.0;
+  for (int i0 = tid; i0 < n; i0 += 8 * 256) {
+    double t8[8][D];
 #pragma unroll
-        for (int q = 0; q < kSV32; q++) {
-          v[q] = op5<float, kSV32>(R, q, n);
-          if (q < n) acc = acc + (double)v[q] * (double)R.c[q];
-        }
-        stv<float, kSV32, false>(w.at(i, j, k), n, v);
-      });
-      store_partial(acc, part + (size_t)t * kPart, sh);
-      continue;
+    for (int u = 0; u < 8; u++) {
+      const int i = i0 + u * 256;
+#pragma unroll
+      for (int k = 0; k < D; k++) t8[u][k] = i < n ? part[(first + k) * np + t0 + i] : 0.0;
     }
-    if (d.kind == OPSMI_SOLVE_HEAT3D) {
-      __syncthreads();  // LDS of the previous tile fully read
-      acc = heat3_column_v<kSV, false, true, kWavesPerBlock, 1>(lds.d, P(d.w, d), Ptr<double>{nullptr, 0, 0},
-                                                                 PC(d.kx, d), PC(d.ky, d), PC(d.kz, d), PC(d.p, d),
-                                                                 d.rx, d.ry, d.rz, b.x0, b.y0, d.nx, d.ny, b.z0,
-                                                                 b.z1);
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (i0 + u * 256 < n)
+#pragma unroll
+        for (int k = 0; k < D; k++) acc[k] = acc[k] + t8[u][k];
+  }
+  block_reduce<double, OPS_INC, D>(acc, sh);
+}
+
+// The CG scalars after an update whose sums are sum[]: iteration count, beta
+// and stop test.  Mixed solves follow the refinement loop of the FP64-IR /
+// FP32-PCG solver:
+//   PH_RESID: residual r, |r|/|f| <= tol stops; else the inner solve starts
+//             with rz and its stop threshold max(inner_tol, tol / (2 relres)) |rr_0|
+//   PH_INNER: stop the inner solve at its threshold (the next sweep corrects
+//             x), else b = (float)(rzn / rz) and p = Mi rr + b p
+__device__ __forceinline__ void advance(SolveStat &q, const SolveDev &d, const double *sum) {
+  q.pending = 0;
+  if (!d.mixed) {
+    const double rrn = sum[0];
+    q.beta = rrn / q.rro;
+    q.rro = rrn;
+    q.iters = q.iters + 1;
+    if (sqrt(rrn) <= q.stop) q.done = 1;
+    else if (q.iters >= q.max_iters) q.done = 2;
+    return;
+  }
+  if (q.phase == PH_INNER) {
+    const double rzn = sum[0], rrn = sum[1];
+    q.iters = q.iters + 1;
+    q.rro = rrn;
+    if (sqrt(rrn) <= q.istop) {
+      q.phase = d.kind == OPSMI_SOLVE_HEAT3D ? PH_CORR : PH_RESID;
+      q.outer = q.outer + 1;
+    } else if (q.iters >= q.max_iters) {
+      q.done = 2;
     } else {
-      const Ptr<const double> p = PC(d.p, d);
-      const Ptr<double> w = P(d.w, d);
-      tile_groups<kSV>(d, b, [&](int x, int y, int z, int n) {
-        Row5<double, kSV> R;
-        load5<double, kSV>(p, x, y, n, R);
-        double v[kSV];
-#pragma unroll
-        for (int q = 0; q < kSV; q++) {
-          v[q] = op5<double, kSV>(R, q, n);
-          if (q < n) acc = acc + v[q] * R.c[q];
-        }
-        stv<double, kSV, false>(w.at(x, y, z), n, v);
-      });
+      q.beta = (double)(float)(rzn / q.rz);
+      q.rz = rzn;
+      q.axpby = 1;
     }
-    store_partial(acc, part + (size_t)t * kPart, sh);
+    return;
+  }
+  const double rrd = sum[0];
+  if (q.outer == 0) {
+    q.fn = sqrt(rrd);
+    q.rr0 = rrd;
+  }
+  q.rro = rrd;
+  const double rel = sqrt(rrd) / q.fn;
+  if (rel <= q.tol) q.done = 1;
+  else if (q.outer >= q.max_outer) q.done = 2;
+  else {
+    q.rz = sum[1];
+    q.istop = fmax(q.inner_tol, 0.5 * q.tol / rel) * sqrt(sum[2]);
+    q.phase = PH_INNER;
+    q.axpby = 0;
   }
 }
 
-__global__ __launch_bounds__(256) void sk_update(const SolveDev *S, const SolveStat *st, const int2 *tiles,
-                                                 const int *ntiles, double *part) {
-  __shared__ double sh[16][1];
-  __shared__ double sh3[16][3];
+// what a launch's workgroups need of their solve's scalars
+struct Step {
+  double a, b;   // p_new = a p + b r
+  double alpha;  // u += alpha p_new, r -= alpha w (update)
+  int done, phase;
+};
+__device__ __forceinline__ Step step_of(const SolveStat &q, const SolveDev &d) {
+  Step c;
+  c.a = q.beta;
+  c.b = 1.0;
+  if (d.mixed) {
+    // p = Mi rr + b p, or p as the residual pass left it
+    c.a = q.axpby ? q.beta : 1.0;
+    c.b = q.axpby ? (d.kind == OPSMI_SOLVE_HEAT3D ? 1.0 : 0.25) : 0.0;
+  }
+  c.alpha = 0.0;
+  c.done = q.done;
+  c.phase = q.phase;
+  return c;
+}
+
+// LDS of an iteration launch: sums being folded, the step all threads read,
+// and the tile's own sums
+struct IterLds {
+  double fold[16][3];
+  double one[16][1];
+  double tile3[16][3];
+  double tile1[16][1];
+  Step step;
+};
+
+// the new scalars in sweep (folds a pending update's sums) and in update
+// (folds p.w); all threads of the workgroup call it, the solve's first tile
+// stores the scalars
+__device__ __forceinline__ Step sweep_step(IterLds &L, const SolveDev &d, const SolveStat &in, SolveStat &out,
+                                           const double *part, size_t np, bool first_of_solve) {
+  const bool pending = in.pending != 0;
+  double sum[3] = {0.0, 0.0, 0.0};
+  if (pending) {
+    if (d.mixed) {
+      fold_partials<3>(part, np, 0, d.tile0, d.ntiles, sum, L.fold);
+    } else {
+      double s1[1];
+      fold_partials<1>(part, np, 0, d.tile0, d.ntiles, s1, L.one);
+      sum[0] = s1[0];
+    }
+  }
+  if (threadIdx.x == 0 && threadIdx.y == 0) {
+    SolveStat q = in;
+    if (pending) advance(q, d, sum);
+    L.step = step_of(q, d);
+    if (first_of_solve) out = q;
+  }
+  __syncthreads();
+  return L.step;
+}
+__device__ __forceinline__ Step update_step(IterLds &L, const SolveDev &d, const SolveStat &in, SolveStat &out,
+                                            const double *part, size_t np, bool first_of_solve) {
+  double pw[1] = {0.0};
+  const bool inner = !d.mixed || in.phase == PH_INNER;
+  if (inner) fold_partials<1>(part, np, 3, d.tile0, d.ntiles, pw, L.one);
+  if (threadIdx.x == 0 && threadIdx.y == 0) {
+    SolveStat q = in;
+    Step c = step_of(q, d);
+    if (inner) {
+      q.pw = pw[0];
+      q.alpha = d.mixed ? (double)(float)(q.rz / pw[0]) : q.rro / pw[0];
+      c.alpha = q.alpha;
+    }
+    // a heat solve's correction has no sums: its residual comes next
+    q.pending = q.phase == PH_CORR ? 0 : 1;
+    if (q.phase == PH_CORR) q.phase = PH_RESID;
+    L.step = c;
+    if (first_of_solve) out = q;
+  }
+  __syncthreads();
+  return L.step;
+}
+
+// V points of a row with their neighbours in the rows below and above and to
+// the left and right, at element offset o.  Loads are whole vectors whatever
+// part of them lies inside the solve: a vector starts on its own size, so it
+// never leaves the field's allocation, and what lies past the last point is
+// the zero halo or padding.
+template <class T, int V>
+struct Star {
+  T c[V], dn[V], up[V], l, r;
+  __device__ __forceinline__ void load(const T *p, long o, long sy) {
+    ldv<T, V>(p + o, V, c);
+    ldv<T, V>(p + o - sy, V, dn);
+    ldv<T, V>(p + o + sy, V, up);
+    l = p[o - 1];
+    r = p[o + V];
+  }
+  // this = a this + b h
+  __device__ __forceinline__ void combine(const Star &h, T a, T b) {
+#pragma unroll
+    for (int j = 0; j < V; j++) {
+      c[j] = a * c[j] + b * h.c[j];
+      dn[j] = a * dn[j] + b * h.dn[j];
+      up[j] = a * up[j] + b * h.up[j];
+    }
+    l = a * l + b * h.l;
+    r = a * r + b * h.r;
+  }
+};
+
+// w = A (a p + b r) of the 2D operator over a tile.  start() issues the first
+// row's loads (before the scalars are known), run() keeps the next row's in
+// flight while a row is computed.
+template <class T, int V>
+struct Sweep5 {
+  const SolveDev &d;
+  const T *p, *r;
+  long sy, xo;
+  int x, y0, n;
+  Star<T, V> P, R;
+  __device__ __forceinline__ Sweep5(const SolveDev &d_, const TileBox &b, const T *p_, const T *r_, long sy_)
+      : d(d_), p(p_), r(r_), sy(sy_) {
+    x = b.x0 + V * (int)threadIdx.x;
+    y0 = b.y0 + (int)threadIdx.y;
+    n = max(0, min(V, d.nx - x));
+    xo = n > 0 ? x : 0;
+  }
+  __device__ __forceinline__ long at(int y) const { return xo + (long)min(y, d.ny - 1) * sy; }
+  __device__ __forceinline__ void start() {
+    P.load(p, at(y0), sy);
+    R.load(r, at(y0), sy);
+  }
+  __device__ __forceinline__ double run(T a, T bb, T *w) {
+    double acc = 0.0;
+    for (int i = 0; i < d.chunk; i++) {
+      const int y = y0 + kWavesPerBlock * i;
+      Star<T, V> C = P;
+      C.combine(R, a, bb);
+      if (i + 1 < d.chunk) {
+        P.load(p, at(y + kWavesPerBlock), sy);
+        R.load(r, at(y + kWavesPerBlock), sy);
+      }
+      const int m = y < d.ny ? n : 0;
+      T v[V];
+#pragma unroll
+      for (int j = 0; j < V; j++) {
+        const T xm = j == 0 ? C.l : C.c[j > 0 ? j - 1 : 0];
+        const T xp = j + 1 < V ? C.c[j + 1 < V ? j + 1 : j] : C.r;
+        v[j] = (T)4.0 * C.c[j] - (xm + xp) - (C.up[j] + C.dn[j]);
+        if (j < m) acc = acc + (double)v[j] * (double)C.c[j];
+      }
+      stv<T, V, false>(w + at(y), m, v);
+    }
+    return acc;
+  }
+};
+
+// A column of the 3D heat operator on q = a p + b r (CHAIN) or on p, marched
+// along z with three planes of q in registers; neighbours along y come from
+// the caches, one plane of loads ahead.  No LDS and no barriers: at these
+// sizes (sides of 32 to 256, mostly in the caches) a plane of the LDS column
+// waited for its loads at a barrier (128^3, 16 planes: 60.8 us an iteration).
+// Arithmetic as HeatColumn (column.h).
+template <class T, int V, bool CHAIN>
+struct HeatMarch {
+  struct Plane {  // loaded for one z: centre of the next plane, rims and coefficients of this one
+    T p[V], ylp[V], yhp[V], xlp, xhp;
+    T r[V], ylr[V], yhr[V], xlr, xhr;
+    T kx[V], ky[V], kyh[V], kzn[V], kxh;
+  };
+  const SolveDev &d;
+  const T *p, *r, *kx, *ky, *kz;
+  long sy, sz, o0;
+  int x, y, z0, z1, n;
+  T pm[V], rm[V], pc[V], rc[V], kzc[V];
+  Plane A;
+  __device__ __forceinline__ HeatMarch(const SolveDev &d_, const TileBox &b, const T *p_, const T *r_, const T *kx_,
+                                       const T *ky_, const T *kz_, long sy_, long sz_)
+      : d(d_), p(p_), r(r_), kx(kx_), ky(ky_), kz(kz_), sy(sy_), sz(sz_) {
+    x = b.x0 + V * (int)threadIdx.x;
+    y = b.y0 + (int)threadIdx.y;
+    z0 = b.z0;
+    z1 = b.z1;
+    n = y < d.ny ? max(0, min(V, d.nx - x)) : 0;
+    o0 = (x < d.nx ? x : 0) + (long)min(y, d.ny - 1) * sy;
+  }
+  __device__ __forceinline__ void load(int z, Plane &A) const {
+    const long o = o0 + (long)z * sz;
+    ldv<T, V>(p + o + sz, V, A.p);
+    ldv<T, V>(p + o - sy, V, A.ylp);
+    ldv<T, V>(p + o + sy, V, A.yhp);
+    A.xlp = p[o - 1];
+    A.xhp = p[o + V];
+    if constexpr (CHAIN) {
+      ldv<T, V>(r + o + sz, V, A.r);
+      ldv<T, V>(r + o - sy, V, A.ylr);
+      ldv<T, V>(r + o + sy, V, A.yhr);
+      A.xlr = r[o - 1];
+      A.xhr = r[o + V];
+    }
+    ldv<T, V>(kx + o, V, A.kx);
+    ldv<T, V>(ky + o, V, A.ky);
+    ldv<T, V>(ky + o + sy, V, A.kyh);
+    ldv<T, V>(kz + o + sz, V, A.kzn);
+    A.kxh = kx[o + V];
+  }
+  __device__ __forceinline__ void start() {
+    const long o = o0 + (long)z0 * sz;
+    ldv<T, V>(p + o - sz, V, pm);
+    ldv<T, V>(p + o, V, pc);
+    if constexpr (CHAIN) {
+      ldv<T, V>(r + o - sz, V, rm);
+      ldv<T, V>(r + o, V, rc);
+    }
+    ldv<T, V>(kz + o, V, kzc);
+    load(z0, A);
+  }
+  template <class OUT>
+  __device__ __forceinline__ void run(T a, T b, T rx, T ry, T rz, OUT &out) {
+    auto q = [&](T pv, T rv) {
+      if constexpr (CHAIN) return a * pv + b * rv;
+      else return pv;
+    };
+    if constexpr (CHAIN) {
+#pragma unroll
+      for (int j = 0; j < V; j++) {
+        pm[j] = q(pm[j], rm[j]);
+        pc[j] = q(pc[j], rc[j]);
+      }
+    }
+    for (int z = z0; z < z1; z++) {
+      Plane C = A;
+      if (z + 1 < z1) load(z + 1, A);
+      T pn[V], v[V];
+      const T xl = q(C.xlp, C.xlr), xh = q(C.xhp, C.xhr);
+#pragma unroll
+      for (int j = 0; j < V; j++) pn[j] = q(C.p[j], C.r[j]);
+#pragma unroll
+      for (int j = 0; j < V; j++) {
+        const T pxm = j == 0 ? xl : pc[j > 0 ? j - 1 : 0];
+        const T pxp = j + 1 < V ? pc[j + 1 < V ? j + 1 : j] : xh;
+        const T kxn = j + 1 < V ? C.kx[j + 1 < V ? j + 1 : j] : C.kxh;
+        const T pym = q(C.ylp[j], C.ylr[j]), pyp = q(C.yhp[j], C.yhr[j]);
+        v[j] = ((T)1.0 + ry * (C.kyh[j] + C.ky[j]) + rx * (kxn + C.kx[j]) + rz * (C.kzn[j] + kzc[j])) * pc[j] -
+               ry * (C.kyh[j] * pyp + C.ky[j] * pym) - rx * (kxn * pxp + C.kx[j] * pxm) -
+               rz * (C.kzn[j] * pn[j] + kzc[j] * pm[j]);
+      }
+      out(x, y, z, n, v, pc);
+#pragma unroll
+      for (int j = 0; j < V; j++) {
+        pm[j] = pc[j];
+        pc[j] = pn[j];
+        kzc[j] = C.kzn[j];
+      }
+    }
+  }
+};
+
+// x = x + (double) e over a tile
+template <int V>
+__device__ __forceinline__ void correct_tile(const SolveDev &d, const TileBox &b) {
+  const Ptr<double> x = P(d.u, d);
+  const Ptr<const float> ev = PF32C(d.e32, d);
+  tile_groups<V>(d, b, [&](int i, int j, int k, int n) {
+    double xv[V];
+    float evv[V];
+    ldv<double, V>(x.at(i, j, k), n, xv);
+    ldv<float, V>(ev.at(i, j, k), n, evv);
+#pragma unroll
+    for (int q = 0; q < V; q++) xv[q] = xv[q] + (double)evv[q];
+    stv<double, V, false>(x.at(i, j, k), n, xv);
+  });
+}
+
+// Both launches: latency-bound on small solves (a tile entry, its solve and
+// the partials are loaded one after the other, then two block reductions:
+// 5.2 us a launch at 64^2), bandwidth-bound on large ones.  A tile's first
+// loads are issued before its solve's sums are folded.  Microseconds per CG
+// iteration of one solve alone, five launches and now:
+//   2D 64^2 17.8 and 12.5, 512^2 19.6 and 14.7, 1000^2 28.0 and 24.0,
+//   2000^2 76.5 and 63.7 (5.0 TB/s of 80 bytes a point); 3D 64^3 24.7 and
+//   17.9, 128^3 60.8 and 47.8; FP32-inner 2D 1000^2 25.0 and 19.4
+__global__ __launch_bounds__(256) void sk_sweep(const SolveDev *__restrict__ S, const SolveStat *__restrict__ in,
+                                                SolveStat *__restrict__ out, const int2 *__restrict__ tiles,
+                                                const int *__restrict__ ntiles, double *part, size_t np) {
+  __shared__ IterLds L;
   const int nt = *ntiles;
   for (int t = first_tile(nt); t < nt; t += (int)gridDim.x) {
-    const int2 e = tiles[t];
-    if (st[e.x].done) continue;
-    const SolveDev d = S[e.x];
-    if (d.mixed) {
-      // 2D Poisson: Jacobi, 1 / diag of the 5-point operator; 3D heat: none
-      const bool heat = d.kind == OPSMI_SOLVE_HEAT3D;
-      const float mi = heat ? 1.0f : 0.25f;
-      // a heat solve's residual pass ran in calc_w (its sums are in place)
-      if (heat && st[e.x].phase == PH_RESID) continue;
-      const Ptr<float> ev = PF32(d.e32, d), rr = PF32(d.r32, d), p = PF32(d.p32, d), w = PF32(d.w32, d);
-      double acc[3] = {0.0, 0.0, 0.0};
-      if (st[e.x].phase == PH_INNER) {
-        // e += a p ; rr -= a w ; (rr . Mi rr, rr . rr) in FP64
-        const float a = (float)st[e.x].alpha;
-        // V: the solve's points per lane (kSV32 for 2D Poisson, kSV for 3D heat)
-        auto inner = [&](auto vt) {
-          constexpr int V = decltype(vt)::value;
-          tile_groups<V>(d, tile_box(d, e.y), [&](int i, int j, int k, int n) {
-            float evv[V], rv[V], pv[V], wv[V];
-            ldv<float, V>(ev.at(i, j, k), n, evv);
-            ldv<float, V>(rr.at(i, j, k), n, rv);
-            ldv<float, V>(p.at(i, j, k), n, pv);
-            ldv<float, V>(w.at(i, j, k), n, wv);
-#pragma unroll
-            for (int q = 0; q < V; q++) {
-              evv[q] = evv[q] + a * pv[q];
-              rv[q] = rv[q] - a * wv[q];
-              const float z = mi * rv[q];
-              if (q < n) {
-                acc[0] = acc[0] + (double)rv[q] * (double)z;
-                acc[1] = acc[1] + (double)rv[q] * (double)rv[q];
-              }
-            }
-            stv<float, V, false>(ev.at(i, j, k), n, evv);
-            stv<float, V, false>(rr.at(i, j, k), n, rv);
-          });
-        };
-        if (d.sv == kSV32) inner(std::integral_constant<int, kSV32>{});
-        else inner(std::integral_constant<int, kSV>{});
+    const int s = __builtin_amdgcn_readfirstlane(tiles[t].x), li = __builtin_amdgcn_readfirstlane(tiles[t].y);
+    const SolveDev &d = S[s];
+    if (in[s].done) {
+      if (li == 0 && threadIdx.x == 0 && threadIdx.y == 0) out[s] = in[s];
+      continue;
+    }
+    const TileBox b = tile_box(d, li);
+    __syncthreads();  // the previous tile's sums have been read
+    if (!d.mixed) {
+      double acc;
+      if (d.kind == OPSMI_SOLVE_HEAT3D) {
+        HeatMarch<double, kSV, true> m(d, b, d.p, d.r, d.kx, d.ky, d.kz, d.sy, d.sz);
+        m.start();
+        const Step c = sweep_step(L, d, in[s], out[s], part, np, li == 0);
+        if (c.done) continue;
+        const Ptr<double> w = P(d.w, d);
+        HeatOutW<double, kSV, false> o{w};
+        m.run(c.a, c.b, d.rx, d.ry, d.rz, o);
+        acc = o.acc;
       } else {
-        // FP64 residual r = f - A x, then the inner start from it:
-        // rr = (float) r, e = 0, p = Mi rr; (r.r, rr . Mi rr, rr . rr).
-        // Runs once per correction: the tile is covered in halves of 64 kSV
-        // points (two doubles per lane, fewer registers for the kernel).
-        const Ptr<const double> x = PC(d.u, d), f = PC(d.f, d);
-        TileBox bh = tile_box(d, e.y);
-        for (int h = 0; h < kSV32 / kSV; h++, bh.x0 += kWave * kSV)
+        Sweep5<double, kSV> m(d, b, d.p, d.r, d.sy);
+        m.start();
+        const Step c = sweep_step(L, d, in[s], out[s], part, np, li == 0);
+        if (c.done) continue;
+        acc = m.run(c.a, c.b, d.w);
+      }
+      store_partial(acc, part + 3 * np + t, L.tile1);
+      continue;
+    }
+    if (d.kind == OPSMI_SOLVE_HEAT3D) {
+      HeatMarch<float, kSV, true> m(d, b, d.p32, d.r32, d.kx32, d.ky32, d.kz32, d.sy32, d.sz32);
+      m.start();
+      const Step c = sweep_step(L, d, in[s], out[s], part, np, li == 0);
+      if (c.done) continue;
+      if (c.phase == PH_CORR) {
+        correct_tile<kSV>(d, b);
+      } else if (c.phase == PH_RESID) {
+        // FP64 residual of the corrected x and the inner start; the sums go
+        // where the update's do (this launch reads none)
+        const Ptr<const double> f = PC(d.f, d);
+        const Ptr<float> rr = PF32(d.r32, d), ev = PF32(d.e32, d), p = PF32(d.p32, d);
+        HeatOutResid o{f, rr, ev, p};
+        HeatMarch<double, kSV, false> md(d, b, d.u, nullptr, d.kx, d.ky, d.kz, d.sy, d.sz);
+        md.start();
+        md.run(1.0, 0.0, d.rx, d.ry, d.rz, o);
+        block_reduce<double, OPS_INC, 3>(o.acc, L.tile3);
+        if (threadIdx.x == 0 && threadIdx.y == 0) {
+          part[t] = o.acc[0];
+          part[np + t] = o.acc[1];
+          part[2 * np + t] = o.acc[2];
+        }
+      } else {
+        const Ptr<float> w = PF32(d.w32, d);
+        HeatOutW<float, kSV, false> o{w};
+        m.run((float)c.a, (float)c.b, (float)d.rx, (float)d.ry, (float)d.rz, o);
+        store_partial(o.acc, part + 3 * np + t, L.tile1);
+      }
+    } else {
+      Sweep5<float, kSV32> m(d, b, d.p32, d.r32, d.sy32);
+      m.start();
+      const Step c = sweep_step(L, d, in[s], out[s], part, np, li == 0);
+      if (c.done) continue;
+      if (c.phase == PH_RESID) {
+        // the correction (pointwise; the residual follows in sk_update once
+        // every tile has applied it)
+        correct_tile<kSV32>(d, b);
+      } else {
+        const double acc = m.run((float)c.a, (float)c.b, d.w32);
+        store_partial(acc, part + 3 * np + t, L.tile1);
+      }
+    }
+  }
+}
+
+// p = a p + b r ; u += alpha p ; r -= alpha w over a tile, sums of r r (and,
+// MIXED, of r.Mi r and r.r).  start() issues the first group's loads.
+template <class T, int V, bool MIXED>
+struct UpdateTile {
+  const SolveDev &d;
+  T *u, *p, *r;
+  const T *w;
+  long sy, sz, xo;
+  int y0, z0, n, groups;
+  bool heat;
+  T uv[V], pv[V], rv[V], wv[V];
+  __device__ __forceinline__ UpdateTile(const SolveDev &d_, const TileBox &b, T *u_, T *p_, T *r_, const T *w_,
+                                        long sy_, long sz_)
+      : d(d_), u(u_), p(p_), r(r_), w(w_), sy(sy_), sz(sz_) {
+    const int x = b.x0 + V * (int)threadIdx.x;
+    heat = d.kind == OPSMI_SOLVE_HEAT3D;
+    y0 = b.y0 + (int)threadIdx.y;
+    z0 = b.z0;
+    n = max(0, min(V, d.nx - x));
+    xo = n > 0 ? x : 0;
+    groups = heat ? b.z1 - b.z0 : d.chunk;
+  }
+  __device__ __forceinline__ int row(int i) const { return heat ? y0 : y0 + kWavesPerBlock * i; }
+  __device__ __forceinline__ long at(int i) const {
+    return xo + (long)min(row(i), d.ny - 1) * sy + (heat ? (long)(z0 + i) * sz : 0);
+  }
+  __device__ __forceinline__ void load(int i) {
+    const long o = at(i);
+    ldv<T, V>(u + o, V, uv);
+    ldv<T, V>(p + o, V, pv);
+    ldv<T, V>(r + o, V, rv);
+    ldv<T, V>(w + o, V, wv);
+  }
+  __device__ __forceinline__ void run(T a, T b, T alpha, T mi, double (&acc)[3]) {
+    for (int i = 0; i < groups; i++) {
+      const int m = row(i) < d.ny ? n : 0;
+      const long o = at(i);
+      T un[V], pn[V], rn[V];
+#pragma unroll
+      for (int q = 0; q < V; q++) {
+        pn[q] = a * pv[q] + b * rv[q];
+        un[q] = uv[q] + alpha * pn[q];
+        rn[q] = rv[q] - alpha * wv[q];
+        if (q < m) {
+          if constexpr (MIXED) {
+            const T z = mi * rn[q];
+            acc[0] = acc[0] + (double)rn[q] * (double)z;
+            acc[1] = acc[1] + (double)rn[q] * (double)rn[q];
+          } else {
+            acc[0] = acc[0] + rn[q] * rn[q];
+          }
+        }
+      }
+      if (i + 1 < groups) load(i + 1);
+      stv<T, V, false>(u + o, m, un);
+      stv<T, V, false>(p + o, m, pn);
+      stv<T, V, false>(r + o, m, rn);
+    }
+  }
+};
+
+// the inner FP32 step of a mixed solve, V points per lane
+template <int V>
+__device__ __forceinline__ void update_inner(IterLds &L, const SolveDev &d, const TileBox &b, const SolveStat &in,
+                                             SolveStat &out, const double *part, size_t np, bool first_of_solve,
+                                             float mi, double (&acc)[3]) {
+  UpdateTile<float, V, true> m(d, b, d.e32, d.p32, d.r32, d.w32, d.sy32, d.sz32);
+  m.load(0);
+  const Step c = update_step(L, d, in, out, part, np, first_of_solve);
+  m.run((float)c.a, (float)c.b, (float)c.alpha, mi, acc);
+}
+
+__global__ __launch_bounds__(256) void sk_update(const SolveDev *__restrict__ S, const SolveStat *__restrict__ in,
+                                                 SolveStat *__restrict__ out, const int2 *__restrict__ tiles,
+                                                 const int *__restrict__ ntiles, double *part, size_t np) {
+  __shared__ IterLds L;
+  const int nt = *ntiles;
+  for (int t = first_tile(nt); t < nt; t += (int)gridDim.x) {
+    const int s = __builtin_amdgcn_readfirstlane(tiles[t].x), li = __builtin_amdgcn_readfirstlane(tiles[t].y);
+    const SolveDev &d = S[s];
+    if (in[s].done) {
+      if (li == 0 && threadIdx.x == 0 && threadIdx.y == 0) out[s] = in[s];
+      continue;
+    }
+    const TileBox b = tile_box(d, li);
+    double acc[3] = {0.0, 0.0, 0.0};
+    __syncthreads();  // the previous tile's sums have been read
+    if (!d.mixed) {
+      UpdateTile<double, kSV, false> m(d, b, d.u, d.p, d.r, d.w, d.sy, d.sz);
+      m.load(0);
+      const Step c = update_step(L, d, in[s], out[s], part, np, li == 0);
+      m.run(c.a, c.b, c.alpha, 1.0, acc);
+      store_partial(acc[0], part + t, L.tile1);
+      continue;
+    }
+    // 2D Poisson: Jacobi, 1 / diag of the 5-point operator; 3D heat: none
+    const bool heat = d.kind == OPSMI_SOLVE_HEAT3D;
+    const float mi = heat ? 1.0f : 0.25f;
+    const int phase = in[s].phase;
+    if (phase == PH_INNER) {
+      if (d.sv == kSV32) update_inner<kSV32>(L, d, b, in[s], out[s], part, np, li == 0, mi, acc);
+      else update_inner<kSV>(L, d, b, in[s], out[s], part, np, li == 0, mi, acc);
+    } else {
+      update_step(L, d, in[s], out[s], part, np, li == 0);
+      if (heat) continue;  // its correction and residual ran in the sweep
+      // FP64 residual r = f - A x, then the inner start from it:
+      // rr = (float) r, e = 0, p = Mi rr; (r.r, rr . Mi rr, rr . rr).
+      // Runs once per correction: the tile is covered in halves of 64 kSV
+      // points (two doubles per lane, fewer registers for the kernel).
+      const Ptr<float> ev = PF32(d.e32, d), rr = PF32(d.r32, d), p = PF32(d.p32, d);
+      const Ptr<const double> x = PC(d.u, d), f = PC(d.f, d);
+      TileBox bh = b;
+      for (int h = 0; h < kSV32 / kSV; h++, bh.x0 += kWave * kSV)
         tile_groups<kSV>(d, bh, [&](int i, int j, int k, int n) {
           Row5<double, kSV> R;
           load5<double, kSV>(x, i, j, n, R);
@@ -415,184 +811,32 @@ __global__ __launch_bounds__(256) void sk_update(const SolveDev *S, const SolveS
           stv<float, kSV, false>(rr.at(i, j, k), n, q32);
           stv<float, kSV, false>(p.at(i, j, k), n, z32);
         });
-      }
-      store_partials<3>(acc, part + (size_t)t * kPart, sh3);
-      continue;
     }
-    const double alpha = st[e.x].alpha;
-    const Ptr<double> u = P(d.u, d), r = P(d.r, d);
-    const Ptr<const double> p = PC(d.p, d), w = PC(d.w, d);
-    double acc = 0.0;
-    tile_groups<kSV>(d, tile_box(d, e.y), [&](int x, int y, int z, int n) {
-      double uv[kSV], rv[kSV], pv[kSV], wv[kSV];
-      ldv<double, kSV>(u.at(x, y, z), n, uv);
-      ldv<double, kSV>(r.at(x, y, z), n, rv);
-      ldv<double, kSV>(p.at(x, y, z), n, pv);
-      ldv<double, kSV>(w.at(x, y, z), n, wv);
-#pragma unroll
-      for (int q = 0; q < kSV; q++) {
-        uv[q] = uv[q] + alpha * pv[q];
-        rv[q] = rv[q] - alpha * wv[q];
-        if (q < n) acc = acc + rv[q] * rv[q];
-      }
-      stv<double, kSV, false>(u.at(x, y, z), n, uv);
-      stv<double, kSV, false>(r.at(x, y, z), n, rv);
-    });
-    store_partial(acc, part + (size_t)t * kPart, sh);
+    block_reduce<double, OPS_INC, 3>(acc, L.tile3);
+    if (threadIdx.x == 0 && threadIdx.y == 0) {
+      part[t] = acc[0];
+      part[np + t] = acc[1];
+      part[2 * np + t] = acc[2];
+    }
   }
 }
 
-__global__ __launch_bounds__(256) void sk_axpby(const SolveDev *S, const SolveStat *st, const int2 *tiles,
-                                                const int *ntiles) {
-  const int nt = *ntiles;
-  for (int t = first_tile(nt); t < nt; t += (int)gridDim.x) {
-    const int2 e = tiles[t];
-    if (st[e.x].done) continue;
-    const SolveDev d = S[e.x];
-    if (d.mixed) {
-      // p = Mi rr + b p, unless the inner solve just stopped or started;
-      // a heat solve whose inner solve just stopped applies x += e here
-      const int ax = st[e.x].axpby;
-      if (!ax) continue;
-      if (ax == 2) {
-        const Ptr<double> x = P(d.u, d);
-        const Ptr<const float> ev = PF32C(d.e32, d);
-        // (3D heat solves only: kSV points per lane)
-        tile_groups<kSV>(d, tile_box(d, e.y), [&](int i, int j, int k, int n) {
-          double xv[kSV];
-          float evv[kSV];
-          ldv<double, kSV>(x.at(i, j, k), n, xv);
-          ldv<float, kSV>(ev.at(i, j, k), n, evv);
-#pragma unroll
-          for (int q = 0; q < kSV; q++) xv[q] = xv[q] + (double)evv[q];
-          stv<double, kSV, false>(x.at(i, j, k), n, xv);
-        });
-        continue;
-      }
-      const float mi = d.kind == OPSMI_SOLVE_HEAT3D ? 1.0f : 0.25f, bf = (float)st[e.x].beta;
-      const Ptr<float> p = PF32(d.p32, d), rr = PF32(d.r32, d);
-      auto pupd = [&](auto vt) {
-        constexpr int V = decltype(vt)::value;
-        tile_groups<V>(d, tile_box(d, e.y), [&](int i, int j, int k, int n) {
-          float pv[V], rv[V];
-          ldv<float, V>(p.at(i, j, k), n, pv);
-          ldv<float, V>(rr.at(i, j, k), n, rv);
-#pragma unroll
-          for (int q = 0; q < V; q++) pv[q] = mi * rv[q] + bf * pv[q];
-          stv<float, V, false>(p.at(i, j, k), n, pv);
-        });
-      };
-      if (d.sv == kSV32) pupd(std::integral_constant<int, kSV32>{});
-      else pupd(std::integral_constant<int, kSV>{});
-      continue;
-    }
-    const double beta = st[e.x].beta;
-    const Ptr<double> p = P(d.p, d);
-    const Ptr<const double> r = PC(d.r, d);
-    tile_groups<kSV>(d, tile_box(d, e.y), [&](int x, int y, int z, int n) {
-      double pv[kSV], rv[kSV];
-      ldv<double, kSV>(p.at(x, y, z), n, pv);
-      ldv<double, kSV>(r.at(x, y, z), n, rv);
-#pragma unroll
-      for (int q = 0; q < kSV; q++) pv[q] = beta * pv[q] + 1.0 * rv[q];
-      stv<double, kSV, false>(p.at(x, y, z), n, pv);
-    });
-  }
-}
-
-// PHASE 0: alpha; PHASE 1: beta, iteration count and stop test
-// Mixed solves follow the refinement loop of the FP64-IR / FP32-PCG solver:
-//   PH_RESID: (x += e), residual r, |r|/|f| <= tol stops; else the inner
-//             solve starts with rz and its stop threshold
-//             max(inner_tol, tol / (2 relres)) |rr_0|
-//   PH_INNER: a = (float)(rz / pw); after the update, stop the inner solve at
-//             its threshold (the next iteration corrects x), else
-//             b = (float)(rzn / rz) and p = Mi rr + b p
-template <int PHASE>
-__global__ __launch_bounds__(256) void sk_fold(const SolveDev *S, SolveStat *st, const double *part) {
+// the last update's sums of a batch of iterations, one workgroup a solve
+__global__ __launch_bounds__(256) void sk_finish(const SolveDev *__restrict__ S, SolveStat *st, const double *part,
+                                                 size_t np) {
   __shared__ double sh[16][3];
   const int s = (int)blockIdx.x;
-  if (!S[s].active || st[s].done) return;
-  const bool mixed = S[s].mixed;
-  const int ph = st[s].phase;
-  if (mixed && PHASE == 0 && ph == PH_RESID) return;  // the correction pass has no sum
-  const int t0 = S[s].tile0, n = S[s].ntiles;
-  double acc[3] = {0.0, 0.0, 0.0};
-  const int nq = mixed && PHASE == 1 ? 3 : 1;
-  // thread i adds partials i, i + 256, ... in that order; eight are loaded
-  // before they are added (eight loads in flight, the same sums)
-  const int nb = (int)blockDim.x;
-  for (int i0 = (int)threadIdx.x; i0 < n; i0 += 8 * nb) {
-    double t8[8][3];
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int i = i0 + u * nb;
-#pragma unroll
-      for (int k = 0; k < 3; k++) t8[u][k] = i < n && k < nq ? part[(size_t)(t0 + i) * kPart + k] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < 8; u++)
-      if (i0 + u * nb < n)
-#pragma unroll
-        for (int k = 0; k < 3; k++)
-          if (k < nq) acc[k] = acc[k] + t8[u][k];
-  }
-  block_reduce<double, OPS_INC, 3>(acc, sh);
-  if (threadIdx.x != 0) return;
-  SolveStat &q = st[s];
-  if (!mixed) {
-    if (PHASE == 0) {
-      q.pw = acc[0];
-      q.alpha = q.rro / acc[0];
-    } else {
-      const double rrn = acc[0];
-      q.beta = rrn / q.rro;
-      q.rro = rrn;
-      q.iters = q.iters + 1;
-      if (sqrt(rrn) <= q.stop) q.done = 1;
-      else if (q.iters >= q.max_iters) q.done = 2;
-    }
-    return;
-  }
-  if (PHASE == 0) {  // PH_INNER
-    q.pw = acc[0];
-    q.alpha = (double)(float)(q.rz / acc[0]);
-    return;
-  }
-  if (ph == PH_INNER) {
-    const double rzn = acc[0], rrn = acc[1];
-    q.iters = q.iters + 1;
-    q.rro = rrn;
-    if (sqrt(rrn) <= q.istop) {
-      q.phase = PH_RESID;
-      q.outer = q.outer + 1;
-      // 2D Poisson: the next calc_w pass applies x += e; 3D heat: this
-      // iteration's axpby pass does, and the next calc_w is the residual
-      q.axpby = S[s].kind == OPSMI_SOLVE_HEAT3D ? 2 : 0;
-    } else if (q.iters >= q.max_iters) {
-      q.done = 2;
-    } else {
-      q.beta = (double)(float)(rzn / q.rz);
-      q.rz = rzn;
-      q.axpby = 1;
-    }
+  if (!S[s].active || st[s].done || !st[s].pending) return;
+  double sum[3];
+  if (S[s].mixed) {
+    fold_partials<3>(part, np, 0, S[s].tile0, S[s].ntiles, sum, sh);
   } else {
-    const double rrd = acc[0];
-    if (q.outer == 0) {
-      q.fn = sqrt(rrd);
-      q.rr0 = rrd;
-    }
-    q.rro = rrd;
-    const double rel = sqrt(rrd) / q.fn;
-    if (rel <= q.tol) q.done = 1;
-    else if (q.outer >= q.max_outer) q.done = 2;
-    else {
-      q.rz = acc[1];
-      q.istop = fmax(q.inner_tol, 0.5 * q.tol / rel) * sqrt(acc[2]);
-      q.phase = PH_INNER;
-      q.axpby = 0;
-    }
+    __shared__ double one[16][1];
+    double s1[1];
+    fold_partials<1>(part, np, 0, S[s].tile0, S[s].ntiles, s1, one);
+    sum[0] = s1[0];
   }
+  if (threadIdx.x == 0) advance(st[s], S[s], sum);
 }
 
 // ------------------------------------------------------------ set-up
@@ -637,14 +881,16 @@ __global__ __launch_bounds__(256) void sk_heat_coefs(SolveDev d) {
 
 // first residual, p = r, partial r.p per tile (grid = the solve's tiles)
 __global__ __launch_bounds__(256) void sk_first_residual(SolveDev d, uint64_t seed, double *part) {
-  __shared__ HeatLdsV<kSV, kWavesPerBlock> lds;
   __shared__ double sh[16][1];
   const int li = (int)blockIdx.x;
   const TileBox b = tile_box(d, li);
-  if (d.kind == OPSMI_SOLVE_HEAT3D)
-    heat3_column_v<kSV, true, false, kWavesPerBlock, 1>(lds, P(d.w, d), P(d.r, d), PC(d.kx, d), PC(d.ky, d),
-                                                         PC(d.kz, d), PC(d.u, d), d.rx, d.ry, d.rz, b.x0, b.y0, d.nx,
-                                                         d.ny, b.z0, b.z1);
+  if (d.kind == OPSMI_SOLVE_HEAT3D) {
+    const Ptr<double> w0 = P(d.w, d), r0 = P(d.r, d);
+    HeatOutInit<double, kSV, false> out{w0, r0};
+    HeatMarch<double, kSV, false> m(d, b, d.u, nullptr, d.kx, d.ky, d.kz, d.sy, d.sz);
+    m.start();
+    m.run(1.0, 0.0, d.rx, d.ry, d.rz, out);
+  }
   const Ptr<double> r = P(d.r, d), p = P(d.p, d);
   const bool poisson = d.kind == OPSMI_SOLVE_POISSON2D;
   double acc = 0.0;
@@ -693,7 +939,7 @@ __global__ void sk_mixed_stat(SolveStat *q, double tol, double inner_tol, int ma
   q->iters = 0;
   q->done = 0;
   q->max_iters = max_iters;
-  q->pad = 0;
+  q->pending = 0;
   q->rz = q->istop = q->fn = 0.0;
   q->tol = tol;
   q->inner_tol = inner_tol;
@@ -717,7 +963,7 @@ __global__ __launch_bounds__(256) void sk_first_fold(SolveStat *q, const double 
     q->iters = 0;
     q->done = 0;
     q->max_iters = max_iters;
-    q->pad = 0;
+    q->pending = 0;
     q->phase = PH_INNER;
     q->outer = 0;
     q->axpby = 0;
@@ -809,7 +1055,7 @@ struct opsmi_server_s {
   char *arena_base = nullptr;
   Arena arena;
   SolveDev *d_solves = nullptr;
-  SolveStat *d_stat = nullptr;
+  SolveStat *d_stat = nullptr;  // two copies of max_slots
   int2 *d_tiles = nullptr;
   int *d_ntiles = nullptr;
   double *d_part = nullptr, *d_setup_part = nullptr;
@@ -871,14 +1117,13 @@ long tiles_of(const opsmi_solve_req &q, int param, int *tx, int *ty) {
 void launch_iterations(opsmi_server S, hipStream_t st, int iters) {
   const dim3 blk(kWave, kWavesPerBlock);
   for (int k = 0; k < iters; k++) {
-    hipLaunchKernelGGL(sk_calc_w, dim3(S->grid), blk, 0, st, S->d_solves, S->d_stat, S->d_tiles, S->d_ntiles,
-                       S->d_part);
-    hipLaunchKernelGGL(sk_fold<0>, dim3(S->max_slots), dim3(256), 0, st, S->d_solves, S->d_stat, S->d_part);
-    hipLaunchKernelGGL(sk_update, dim3(S->grid), blk, 0, st, S->d_solves, S->d_stat, S->d_tiles, S->d_ntiles,
-                       S->d_part);
-    hipLaunchKernelGGL(sk_fold<1>, dim3(S->max_slots), dim3(256), 0, st, S->d_solves, S->d_stat, S->d_part);
-    hipLaunchKernelGGL(sk_axpby, dim3(S->grid), blk, 0, st, S->d_solves, S->d_stat, S->d_tiles, S->d_ntiles);
+    hipLaunchKernelGGL(sk_sweep, dim3(S->grid), blk, 0, st, S->d_solves, S->d_stat, S->d_stat + S->max_slots,
+                       S->d_tiles, S->d_ntiles, S->d_part, S->max_tiles);
+    hipLaunchKernelGGL(sk_update, dim3(S->grid), blk, 0, st, S->d_solves, S->d_stat + S->max_slots, S->d_stat,
+                       S->d_tiles, S->d_ntiles, S->d_part, S->max_tiles);
   }
+  hipLaunchKernelGGL(sk_finish, dim3(S->max_slots), dim3(256), 0, st, S->d_solves, S->d_stat, S->d_part,
+                     S->max_tiles);
 }
 
 // admits the queue head while a slot and memory are free; sets up on device
@@ -1092,13 +1337,13 @@ opsmi_server opsmi_serve_create(size_t hbm_budget, int max_slots, int iters_per_
   OPSMI_HIP(hipMalloc(&S->arena_base, S->budget));
   S->arena.init(S->budget);
   OPSMI_HIP(hipMalloc(&S->d_solves, sizeof(SolveDev) * max_slots));
-  OPSMI_HIP(hipMalloc(&S->d_stat, sizeof(SolveStat) * max_slots));
+  OPSMI_HIP(hipMalloc(&S->d_stat, 2 * sizeof(SolveStat) * max_slots));
   OPSMI_HIP(hipMalloc(&S->d_tiles, sizeof(int2) * S->max_tiles));
   OPSMI_HIP(hipMalloc(&S->d_ntiles, sizeof(int)));
   OPSMI_HIP(hipMalloc(&S->d_part, sizeof(double) * kPart * S->max_tiles));
   OPSMI_HIP(hipMalloc(&S->d_setup_part, sizeof(double) * S->max_tiles));
   OPSMI_HIP(hipHostMalloc((void **)&S->h_stat, sizeof(SolveStat) * max_slots, hipHostMallocDefault));
-  OPSMI_HIP(hipMemsetAsync(S->d_stat, 0, sizeof(SolveStat) * max_slots, S->stream));
+  OPSMI_HIP(hipMemsetAsync(S->d_stat, 0, 2 * sizeof(SolveStat) * max_slots, S->stream));
   S->h_solves.assign(max_slots, SolveDev{});
   S->slot_req.assign(max_slots, -1);
   rebuild_tables(S);

@@ -263,3 +263,34 @@ def test_tile_tables_from_one_tile_to_more_than_the_grid(serve, n):
     ref = O.poisson_cg(2, n, n, 1, O.poisson_rhs(SEED, 2, n, n), max_iters=4, tol=1e-10, nthreads=8)
     assert done["iters"] == ref["iters"]
     assert np.max(np.abs(x - ref["x"])) <= 1e-12 * np.max(np.abs(ref["x"]))
+
+
+@pytest.mark.parametrize("n", [2, 3, 5, 31, 33, 63, 65, 127, 129])
+def test_heat_columns_at_tile_edges(serve, n):
+    # sides around the tile's 128 points, 4 rows and 4 or 16 planes; four CG
+    # iterations.  The conductivity comes from device exp, log and cos (an ulp
+    # or two from the host's), which the solution carries on: 1e-10.
+    S = serve
+    srv = S.Server(budget_bytes=1 << 29, max_slots=2)
+    i = srv.submit(S.HEAT3D, n, seed=SEED, max_iters=4)
+    done, x = srv.run()[i]
+    srv.close()
+    K, rhs = O.heat_inputs(SEED, 3, n, n, n)
+    ref = O.heat_cg(3, n, n, n, K, rhs, max_iters=4, tol=1e-10, nthreads=8)
+    assert done["iters"] == ref["iters"]
+    assert np.max(np.abs(x - ref["u"])) <= 1e-10 * np.max(np.abs(ref["u"]))
+
+
+@pytest.mark.parametrize("kind,n", [(0, 3), (0, 129), (0, 257), (0, 511), (1, 5), (1, 33), (1, 65)])
+def test_mixed_at_tile_edges_equals_fp64(serve, kind, n):
+    # both stop at a relative residual of 1e-10, so they differ by at most the
+    # operator's condition (about (n/2)^2 in 2D, 1e3 for these heat problems)
+    # times that, in practice far less
+    S = serve
+    srv = S.Server(budget_bytes=1 << 29, max_slots=4)
+    a = srv.submit(kind, n, seed=SEED)
+    b = srv.submit(kind, n, seed=SEED, mixed=True)
+    out = srv.run()
+    srv.close()
+    assert out[a][0]["status"] == 1 and out[b][0]["status"] == 1
+    assert np.max(np.abs(out[a][1] - out[b][1])) <= 1e-8 * np.max(np.abs(out[a][1]))
