@@ -86,3 +86,33 @@ def test_halo_transfer_soa_equals_aos(gpu_ops):
         out.append(ops.get_whole(b))
     assert np.array_equal(out[0], out[1])
     assert np.any(out[0] != -1)
+
+
+@pytest.mark.parametrize("dtype,dim,count", [(np.float64, 1, 1), (np.float64, 1, 36), (np.float32, 2, 37),
+                                             (np.int32, 1, 150)])
+def test_halos_of_a_group_act_in_order(gpu_ops, dtype, dim, count):
+    """Boxes anywhere in three dats, many meeting an earlier one's target: the
+    same as one halo after another (numpy), however they are launched."""
+    ops = gpu_ops
+    rng = np.random.RandomState(11 + count)
+    nx, ny, h = 40, 31, 3
+    blk = ops.ops_decl_block(2, "horder")
+    shape = (ny + 2 * h, nx + 2 * h) + ((dim,) if dim > 1 else ())
+    ref = [rng.randint(-1000, 1000, shape).astype(dtype) for _ in range(3)]
+    dats = []
+    for r in ref:
+        dats.append(ops.ops_decl_dat(blk, [nx, ny], [-h, -h], [h, h], dtype, "h", dim=dim))
+        ops.set_whole(dats[-1], r)
+    hs = []
+    for _ in range(count):
+        f, t = rng.randint(3), rng.randint(3)
+        it = [int(rng.randint(1, 9)), int(rng.randint(1, 7))]
+        fb = [int(rng.randint(-h, n + h - i + 1)) for n, i in zip((nx, ny), it)]
+        tb = [int(rng.randint(-h, n + h - i + 1)) for n, i in zip((nx, ny), it)]
+        hs.append(ops.ops_decl_halo(dats[f], dats[t], it, fb, tb, [1, 2], [1, 2]))
+        box = [tuple(slice(b[q] + h, b[q] + h + it[q]) for q in (1, 0)) for b in (fb, tb)]
+        ref[t][box[1]] = ref[f][box[0]].copy()
+    ops.ops_halo_transfer(ops.ops_decl_halo_group(hs))
+    for d, r in zip(dats, ref):
+        assert np.array_equal(ops.get_whole(d), r)
+        ops.ops_free_dat(d)
