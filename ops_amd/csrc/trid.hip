@@ -13,8 +13,8 @@
 //   x_i = d'_i - c'_i x_{i+1}
 // with contraction off, so results equal the CPU restatement bit for bit.
 //
-// PCR (strategy PCR): one workgroup per system held in LDS, log2(n) steps of
-// parallel cyclic reduction (Hockney 1965); a_0 and c_{n-1} are taken as 0.
+// PCR (strategy PCR): log2(n) steps of parallel cyclic reduction (Hockney
+// 1965) in registers and LDS; a_0 and c_{n-1} are taken as 0.
 #include "engine.h"
 
 using namespace opsmi;
@@ -34,7 +34,8 @@ struct LineGeo {
 };
 
 __device__ __forceinline__ long line_offset(const LineGeo &g, long id) {
-  long i0 = id % g.e0, i1 = id / g.e0;
+  // (a 64-bit division takes some hundred instructions)
+  const long i1 = id >> 32 ? id / g.e0 : (long)((unsigned)id / (unsigned)g.e0), i0 = id - i1 * g.e0;
   return i0 * g.s0 + i1 * g.s1;
 }
 
@@ -397,56 +398,141 @@ __global__ __launch_bounds__(64) void k_thomas_x(const T *__restrict__ a, const 
   }
 }
 
-template <class T, bool INC>
-__global__ __launch_bounds__(1024) void k_pcr(const T *__restrict__ a, const T *__restrict__ b,
-                                              const T *__restrict__ c, T *__restrict__ d, T *__restrict__ u,
-                                              LineGeo g) {
-  extern __shared__ unsigned char smem[];
-  T *A = (T *)smem;
-  T *B = A + 2 * g.n;
-  T *C = B + 2 * g.n;
-  T *D = C + 2 * g.n;
-  const long o = line_offset(g, blockIdx.x);
-  const int n = (int)g.n;
-  const int i = threadIdx.x;
-  const long s = g.stride;
-  if (i < n) {
-    A[i] = i == 0 ? (T)0 : a[o + i * s];
-    B[i] = b[o + i * s];
-    C[i] = i == n - 1 ? (T)0 : c[o + i * s];
-    D[i] = d[o + i * s];
+// PCR.  A workgroup takes S neighbouring systems of n rows; J threads share a
+// system, thread j holding rows j, j + J, ... (at most ROWS) in registers.
+// The steps of distance below J find their neighbours through LDS, those of
+// J and above in the thread's own registers.  Lanes run along the systems for
+// solves along y and z and along the rows for solves along x (ALONG), so a
+// load takes whole segments either way (one workgroup per system read 8 bytes
+// of every 128-byte line along y and z).  Bounded by vector arithmetic, 62
+// instructions a row and step, two divisions among them: sharing their
+// reciprocals (same quotients by Markstein's correction) saved nothing after
+// its range checks.  Microseconds along x / y / z, before and now: 256^3
+// 346 / 775 / 900 and 354 / 405 / 365, 200 x 130 x 97 63 / 118 / 148 and
+// 65 / 60 / 52.  Two rows a thread; 4 and 8 rows took 387 / 403 / 389 and
+// 384 / 417 / 388 at 256^3, so longer systems only, which would otherwise
+// leave a workgroup one system, take 4.  The operations of a row are the
+// algorithm's, in its order.
+constexpr int kPcrShort = 256;  // rows up to which a thread takes two
+
+template <class T>
+struct PcrRow {
+  T a, b, c, d;
+};
+
+// one step of a row: lo, hi its neighbours where they exist
+template <class T>
+__device__ __forceinline__ PcrRow<T> pcr_step(const PcrRow<T> &x, bool lo, const PcrRow<T> &l, bool hi,
+                                              const PcrRow<T> &h) {
+  const T k1 = lo ? x.a / l.b : (T)0;
+  const T k2 = hi ? x.c / h.b : (T)0;
+  T bv = x.b, dv = x.d;
+  if (lo) {
+    bv = bv - l.c * k1;
+    dv = dv - l.d * k1;
   }
-  __syncthreads();
-  int cur = 0;
-  for (int st = 1; st < n; st *= 2) {
-    const int nx = cur ^ n;  // offset of the other buffer half (0 or n)
-    if (i < n) {
-      const T *Ac = A + cur, *Bc = B + cur, *Cc = C + cur, *Dc = D + cur;
-      const bool lo = i - st >= 0, hi = i + st < n;
-      const T k1 = lo ? Ac[i] / Bc[i - st] : (T)0;
-      const T k2 = hi ? Cc[i] / Bc[i + st] : (T)0;
-      T bv = Bc[i], dv = Dc[i];
-      if (lo) {
-        bv = bv - Cc[i - st] * k1;
-        dv = dv - Dc[i - st] * k1;
+  if (hi) {
+    bv = bv - h.a * k2;
+    dv = dv - h.d * k2;
+  }
+  return PcrRow<T>{lo ? -l.a * k1 : (T)0, bv, hi ? -h.c * k2 : (T)0, dv};
+}
+
+template <class T, bool INC, bool ALONG, int ROWS>
+__global__ __launch_bounds__(512) void k_pcr(const T *__restrict__ a, const T *__restrict__ b,
+                                             const T *__restrict__ c, T *__restrict__ d, T *__restrict__ u,
+                                             LineGeo g, int S, int J) {
+  extern __shared__ unsigned char smem[];
+  const int n = (int)g.n, tid = (int)threadIdx.x;
+  const int s = ALONG ? tid / J : tid & (S - 1), j = ALONG ? tid & (J - 1) : tid / S;
+  const long id = (long)xcd_tile(blockIdx.x, gridDim.x) * S + s;
+  const bool live = id < g.count;
+  const long o = live ? line_offset(g, id) : 0;
+  // LDS: rows of a system one after the other, or systems of a row; this
+  // thread's rows are kstep apart in it and gstep apart in memory
+  const int lr = ALONG ? 1 : S, kstep = J * lr, all = n * S;
+  const int at = (ALONG ? s * n : s) + j * lr;
+  typedef vec_t<T, 2> Pair;
+  Pair *L = (Pair *)smem + at;
+  const long q0 = o + j * g.stride, gstep = J * g.stride;
+  PcrRow<T> r[ROWS];
+#pragma unroll
+  for (int k = 0; k < ROWS; k++) {
+    const int i = j + k * J;
+    r[k] = PcrRow<T>{(T)0, (T)1, (T)0, (T)0};
+    if (live && i < n) {
+      const long q = q0 + k * gstep;
+      r[k] = PcrRow<T>{a[q], b[q], c[q], d[q]};
+      if (i == 0) r[k].a = (T)0;
+      if (i == n - 1) r[k].c = (T)0;
+    }
+  }
+  const int top = min(J, n);
+  for (int st = 1; st < top; st *= 2) {
+#pragma unroll
+    for (int k = 0; k < ROWS; k++)
+      if (j + k * J < n) {
+        Pair *p = L + k * kstep;
+        p[0] = Pair{r[k].a, r[k].b};
+        p[all] = Pair{r[k].c, r[k].d};
       }
-      if (hi) {
-        bv = bv - Ac[i + st] * k2;
-        dv = dv - Dc[i + st] * k2;
+    __syncthreads();
+    const int away = st * lr;
+#pragma unroll
+    for (int k = 0; k < ROWS; k++) {
+      const int i = j + k * J;
+      if (i < n) {
+        const bool lo = i >= st, hi = i + st < n;
+        const Pair *l = L + (k * kstep - (lo ? away : 0)), *h = L + (k * kstep + (hi ? away : 0));
+        const Pair l0 = l[0], l1 = l[all], h0 = h[0], h1 = h[all];
+        r[k] = pcr_step(r[k], lo, PcrRow<T>{l0[0], l0[1], l1[0], l1[1]}, hi, PcrRow<T>{h0[0], h0[1], h1[0], h1[1]});
       }
-      A[nx + i] = lo ? -Ac[i - st] * k1 : (T)0;
-      C[nx + i] = hi ? -Cc[i + st] * k2 : (T)0;
-      B[nx + i] = bv;
-      D[nx + i] = dv;
     }
     __syncthreads();
-    cur = nx;
   }
-  if (i < n) {
-    const T x = D[cur + i] / B[cur + i];
-    if (INC) u[o + i * s] = u[o + i * s] + x;
-    else d[o + i * s] = x;
+#pragma unroll
+  for (int m = 1; m < ROWS; m *= 2) {
+    if (m * J >= n) break;
+    PcrRow<T> x[ROWS];
+#pragma unroll
+    for (int k = 0; k < ROWS; k++) {
+      const bool lo = k >= m, hi = k + m < ROWS && j + (k + m) * J < n;
+      const int l = k >= m ? k - m : k, h = k + m < ROWS ? k + m : k;
+      x[k] = pcr_step(r[k], lo, r[l], hi, r[h]);
+    }
+#pragma unroll
+    for (int k = 0; k < ROWS; k++) r[k] = x[k];
   }
+#pragma unroll
+  for (int k = 0; k < ROWS; k++) {
+    const int i = j + k * J;
+    if (live && i < n) {
+      const T x = r[k].d / r[k].b;
+      const long q = q0 + k * gstep;
+      if (INC) u[q] = u[q] + x;
+      else d[q] = x;
+    }
+  }
+}
+
+// threads per system and systems per workgroup
+struct PcrShape {
+  int S, J;
+  size_t lds;
+};
+inline PcrShape pcr_shape(int n, size_t es) {
+  PcrShape p;
+  p.J = 1;
+  while (p.J * (n <= kPcrShort ? 2 : 4) < n) p.J *= 2;
+  // 128 bytes of systems where their rows then fit the 64 KiB of LDS a
+  // workgroup may ask for, at most 512 threads; fewer systems for long ones
+  p.S = (int)(128 / es);
+  const size_t row = 4 * es;  // bytes in LDS
+  while (p.S > 1 && (p.S * p.J > 512 || n * p.S * row > (64u << 10))) p.S /= 2;
+  // short systems: at least four waves a workgroup
+  while (p.S * p.J < 256 && n * p.S * 2 * row <= (40u << 10)) p.S *= 2;
+  p.lds = p.J > 1 ? n * p.S * row : 0;
+  return p;
 }
 
 struct TridScratch {
@@ -568,16 +654,28 @@ void trid_run(int ndim, int solvedim, int *range, ops_dat a, ops_dat b, ops_dat 
   bool pcr = ctx && ctx->strategy == 3;
   if (pcr) {
     if (g.n > 1024) fail(OPS_NOT_IMPLEMENTED, "Tridsolver error: PCR supports systems of at most 1024 rows");
-    int threads = (int)((g.n + 63) / 64 * 64);
-    size_t sm = 8 * g.n * es;
+    const PcrShape ps = pcr_shape((int)g.n, es);
+    const unsigned nb = (unsigned)((g.count + ps.S - 1) / ps.S);
+    const dim3 block((unsigned)(ps.S * ps.J));
     launch([&](hipStream_t s) {
-      if (dt == DT_F64) {
-        if (u) hipLaunchKernelGGL((k_pcr<double, true>), dim3(g.count), dim3(threads), sm, s, (double *)pa, (double *)pb, (double *)pc, (double *)pd, (double *)pu, g);
-        else hipLaunchKernelGGL((k_pcr<double, false>), dim3(g.count), dim3(threads), sm, s, (double *)pa, (double *)pb, (double *)pc, (double *)pd, (double *)pu, g);
-      } else {
-        if (u) hipLaunchKernelGGL((k_pcr<float, true>), dim3(g.count), dim3(threads), sm, s, (float *)pa, (float *)pb, (float *)pc, (float *)pd, (float *)pu, g);
-        else hipLaunchKernelGGL((k_pcr<float, false>), dim3(g.count), dim3(threads), sm, s, (float *)pa, (float *)pb, (float *)pc, (float *)pd, (float *)pu, g);
-      }
+      auto go = [&](auto kern, auto *t) {
+        using T = std::remove_pointer_t<decltype(t)>;
+        hipLaunchKernelGGL(kern, dim3(nb), block, ps.lds, s, (const T *)pa, (const T *)pb, (const T *)pc, (T *)pd,
+                           (T *)pu, g, ps.S, ps.J);
+      };
+      auto rows = [&](auto r, auto *t) {
+        using T = std::remove_pointer_t<decltype(t)>;
+        constexpr int ROWS = decltype(r)::value;
+        const bool x = solvedim == 0;
+        if (u) go(x ? k_pcr<T, true, true, ROWS> : k_pcr<T, true, false, ROWS>, t);
+        else go(x ? k_pcr<T, false, true, ROWS> : k_pcr<T, false, false, ROWS>, t);
+      };
+      auto type = [&](auto *t) {
+        if (g.n <= kPcrShort) rows(std::integral_constant<int, 2>{}, t);
+        else rows(std::integral_constant<int, 4>{}, t);
+      };
+      if (dt == DT_F64) type((double *)nullptr);
+      else type((float *)nullptr);
     });
   } else {
     size_t sb = (size_t)g.n * g.count * es;

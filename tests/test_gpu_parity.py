@@ -690,3 +690,59 @@ def test_stencil27_column_bit_exact(gpu_ops, n):
     assert np.array_equal(ops.ops_dat_fetch_data(o), O.stencil27(nx, ny, nz, ue))
     ops.ops_free_dat(u)
     ops.ops_free_dat(o)
+
+
+def _pcr_numpy(a, b, c, d):
+    """parallel cyclic reduction along the last axis in the arrays' own type,
+    with the operations and order of the kernel and the oracle"""
+    a, b, c, d = (v.copy() for v in (a, b, c, d))
+    n = d.shape[-1]
+    a[..., 0] = 0
+    c[..., n - 1] = 0
+    st = 1
+    while st < n:
+        k1, k2 = np.zeros_like(d), np.zeros_like(d)
+        k1[..., st:] = a[..., st:] / b[..., :-st]
+        k2[..., :-st] = c[..., :-st] / b[..., st:]
+        nb, nd, na, nc = b.copy(), d.copy(), np.zeros_like(d), np.zeros_like(d)
+        nb[..., st:] = nb[..., st:] - c[..., :-st] * k1[..., st:]
+        nd[..., st:] = nd[..., st:] - d[..., :-st] * k1[..., st:]
+        nb[..., :-st] = nb[..., :-st] - a[..., st:] * k2[..., :-st]
+        nd[..., :-st] = nd[..., :-st] - d[..., st:] * k2[..., :-st]
+        na[..., st:] = -a[..., :-st] * k1[..., st:]
+        nc[..., :-st] = -c[..., st:] * k2[..., :-st]
+        a, b, c, d = na, nb, nc, nd
+        st *= 2
+    return d / b
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [(1, 2, 3), (4, 5, 8), (9, 16, 17), (31, 33, 40), (65, 24, 63), (130, 128, 11),
+                               (256, 257, 3), (3, 300, 9), (513, 4, 512), (1024, 3, 2), (5, 2, 1000)])
+def test_pcr_shapes_bit_exact(gpu_ops, dtype, n):
+    """lengths around the rows a thread holds, the threads a system takes and
+    the systems a workgroup takes, along each dimension, in place and _Inc"""
+    ops = gpu_ops
+    rng = np.random.RandomState(5)
+    shape = n[::-1]
+    blk = ops.ops_decl_block(3, "pcrshape")
+    D = {k: ops.ops_decl_dat(blk, list(n), dtype=dtype, name=k) for k in "abcdu"}
+    ctx = ops.TridParams(blk, ops.TridParams.PCR)
+    rg = [0, n[0], 0, n[1], 0, n[2]]
+    # sizes of 1 are edge dimensions of a dat: they hold one point
+    A, Cc = rng.rand(*shape).astype(dtype) - 1, rng.rand(*shape).astype(dtype) - 1
+    B = (abs(A) + abs(Cc) + dtype(0.1) + rng.rand(*shape).astype(dtype)).astype(dtype)
+    X, U = rng.rand(*shape).astype(dtype), rng.rand(*shape).astype(dtype)
+    for k, v in zip("abcdu", (A, B, Cc, X, U)):
+        ops.ops_dat_set_data(D[k], v)
+    for sd in range(3):
+        ax = 2 - sd
+        x = np.moveaxis(_pcr_numpy(*(np.moveaxis(v, ax, -1) for v in (A, B, Cc, X))), -1, ax)
+        U = U + x
+        ops.ops_tridMultiDimBatch_Inc(3, sd, rg, D["a"], D["b"], D["c"], D["d"], D["u"], ctx)
+        assert np.array_equal(ops.ops_dat_fetch_data(D["u"]), U), sd
+        X = np.ascontiguousarray(x)
+        ops.ops_tridMultiDimBatch(3, sd, rg, D["a"], D["b"], D["c"], D["d"], ctx)
+        assert np.array_equal(ops.ops_dat_fetch_data(D["d"]), X), sd
+    for q in D.values():
+        ops.ops_free_dat(q)
