@@ -746,3 +746,37 @@ def test_pcr_shapes_bit_exact(gpu_ops, dtype, n):
         assert np.array_equal(ops.ops_dat_fetch_data(D["d"]), X), sd
     for q in D.values():
         ops.ops_free_dat(q)
+
+
+@pytest.mark.parametrize("n", [(2, 3, 4), (65, 9, 8), (129, 6, 5), (256, 10, 3), (300, 7, 6)])
+def test_preproc_edges_and_remainders(gpu_ops, n):
+    """two points per lane: odd lengths, lengths around a wave's 128 points,
+    rows without 16-byte pitch, and the boundary's own values"""
+    ops = gpu_ops
+    nx, ny, nz = n
+    rng = np.random.RandomState(2)
+    blk = ops.ops_decl_block(3, "preproc_n")
+    names = ["u", "du", "ax", "bx", "cx", "ay", "by", "cy", "az", "bz", "cz"]
+    D = {k: ops.ops_decl_dat(blk, list(n), name=k) for k in names}
+    ext = rng.rand(nz + 2, ny + 2, nx + 2)
+    ops.set_whole(D["u"], ext)
+    for k, v in zip(("nx", "ny", "nz"), n):
+        ops.ops_decl_const(k, 1, "int", v)
+    lam = 0.7
+    ops.ops_decl_const("lambda", 1, "double", lam)
+    s0 = ops.ops_decl_stencil(3, 1, [0, 0, 0], "p0")
+    s7 = ops.ops_decl_stencil(3, 7, [0, 0, 0, 1, 0, 0, -1, 0, 0, 0, 1, 0, 0, -1, 0, 0, 0, 1, 0, 0, -1], "p7")
+    ops.ops_par_loop("preproc_kernel", "preproc", blk, 3, [0, nx, 0, ny, 0, nz],
+                     ops.ops_arg_dat(D["u"], 1, s7, "double", ops.OPS_READ),
+                     *[ops.ops_arg_dat(D[k], 1, s0, "double", ops.OPS_WRITE) for k in names[1:]], ops.ops_arg_idx())
+    c = ext[1:-1, 1:-1, 1:-1]
+    d = lam * (ext[1:-1, 1:-1, :-2] + ext[1:-1, 1:-1, 2:] + ext[1:-1, :-2, 1:-1] + ext[1:-1, 2:, 1:-1] +
+               ext[:-2, 1:-1, 1:-1] + ext[2:, 1:-1, 1:-1] - 6.0 * c)
+    inner = np.zeros(c.shape, bool)
+    inner[1:-1, 1:-1, 1:-1] = True
+    assert np.array_equal(ops.ops_dat_fetch_data(D["du"]), np.where(inner, d, 0.0))
+    for k in names[2:]:
+        v = 1.0 + lam if k[0] == "b" else -0.5 * lam
+        assert np.array_equal(ops.ops_dat_fetch_data(D[k]), np.where(inner, v, 1.0 if k[0] == "b" else 0.0)), k
+    for q in D.values():
+        ops.ops_free_dat(q)
