@@ -14,9 +14,13 @@
 // other workgroup reads, load with the non-temporal hint; p and r, whose
 // edge rows are neighbouring tiles' rims, load without it (TeaLeaf chain at
 // 512^3: 1788 us, against 1820 us with no hints and 1824 us with hints on
-// every centre load).  Lanes past the range end keep to the barriers; a lane with fewer
-// than V points in range loads and stores them one by one, and the lane
-// holding the last point loads the far x rim.
+// every centre load).  A lane or row past the range end loads the last lane's or row's
+// values (and stores nothing), and a lane with fewer than V points in range
+// loads whole vectors all the same, so the loads carry no conditions: a
+// 16-byte vector that starts on a dat's element ends inside its allocation
+// (which is padded by 256 bytes), and what it holds past the range is the far
+// x rim.  (With conditional loads the edge tiles waited for one load after the
+// other: the TeaLeaf chain at 197 x 150 x 131 took 139 us, 66 us so.)
 //
 // Requirements (checked by the launchers): every array's point (x0, y, z)
 // is 16-byte aligned for all rows and planes (row and plane pitches are
@@ -53,6 +57,7 @@ struct ColLane {
   int n;     // points of this lane in range (0..V)
   int cnt;   // points of the tile row in range
   int lye;   // last row in range
+  int lx, ly;  // lane and row whose points it loads: its own, or the last in range
   bool hxl, hxh, hyl, hyh;
 };
 template <int V, int WY = kWavesPerBlock>
@@ -62,6 +67,8 @@ __device__ __forceinline__ ColLane col_lane(int x0, int y0, int xe, int ye) {
   c.cnt = min(kWave * V, xe - x0);
   c.lye = min(WY, ye - y0) - 1;
   c.n = ly <= c.lye ? max(0, min(V, c.cnt - V * lx)) : 0;
+  c.lx = min(lx, (c.cnt - 1) / V);
+  c.ly = min(ly, c.lye);
   c.hxl = lx == 0;
   c.hxh = lx == (c.cnt - 1) / V;
   c.hyl = ly == 0;
@@ -102,6 +109,36 @@ inline ColGrid heat_column_grid(const Range3 &r, int tile_x, int rows) {
   } else {
     g.chunk = 64;
     while (g.chunk > 8 && (long)g.gx * g.gy * ((nz + g.chunk - 1) / g.chunk) < 1024) g.chunk >>= 1;
+  }
+  g.gz = (unsigned)((nz + g.chunk - 1) / g.chunk);
+  return g;
+}
+
+// Launch grid of the columns whose sums need not keep heat_column_grid's
+// grouping (the heat operator's do: its first CG iterations carry the last
+// bit of a sum far at points of extreme conductivity, so their partials stay
+// as they are).  The Poisson columns, and those without a sum, take the planes
+// per workgroup that need the fewest plane steps: a CU works on one
+// 512-thread workgroup at a time (142 to 212 VGPRs), so a grid takes
+// ceil(workgroups / CUs) rounds of its planes and about three planes' worth
+// of start (the planes around the first, and their latency).  At most 64
+// planes, beyond which the workgroups of a round drift apart.  First heat
+// residual at 197 x 150 x 131: 41 us with 22 planes in one round, 50 with 8 in
+// three; FP32 Poisson chain at 400 x 384 x 390: 288 us with 49 planes, 307
+// with 32.
+inline ColGrid column_grid(const Range3 &r, int tile_x, int rows) {
+  ColGrid g = heat_column_grid(r, tile_x, rows);
+  if (getenv("OPSMI_HEAT_ZCHUNK")) return g;
+  const long nz = r.z1 - r.z0;
+  long best = -1;
+  for (long k = (nz + 63) / 64; k <= nz; k++) {
+    const long c = (nz + k - 1) / k, n = (long)g.gx * g.gy * ((nz + c - 1) / c);
+    const long cost = (n + inst().num_cus - 1) / inst().num_cus * (c + 3);
+    if (best < 0 || cost < best) {
+      best = cost;
+      g.chunk = (int)c;
+    }
+    if (c <= 2) break;
   }
   g.gz = (unsigned)((nz + g.chunk - 1) / g.chunk);
   return g;
@@ -180,8 +217,8 @@ struct HeatColumn {
     ly = (int)threadIdx.y;
     c = col_lane<V, WY>(x0, y0, xe, ye);
     if (FULL) c.n = V;
-    x = x0 + V * lx;
-    y = y0 + ly;
+    x = x0 + V * (FULL ? lx : c.lx);
+    y = y0 + (FULL ? ly : c.ly);
     o = V + V * lx;
   }
   __device__ __forceinline__ int n() const { return FULL ? V : c.n; }
@@ -192,19 +229,19 @@ struct HeatColumn {
   // same loads (the compiler then keeps them in flight across the barrier)
   __device__ __forceinline__ void load(int q, Plane &P) const {
     const int qk = min(q, z1 - 1);
-    ldv<T, V>(p.at(x, y, q), n(), P.p);
-    ldv<T, V, true>(Kz.at(x, y, q), n(), P.kz);
-    ldv<T, V, true>(Kx.at(x, y, qk), n(), P.kx);
-    ldv<T, V, true>(Ky.at(x, y, qk), n(), P.ky);
+    ldv<T, V>(p.at(x, y, q), V, P.p);
+    ldv<T, V, true>(Kz.at(x, y, q), V, P.kz);
+    ldv<T, V, true>(Kx.at(x, y, qk), V, P.kx);
+    ldv<T, V, true>(Ky.at(x, y, qk), V, P.ky);
     if (c.hxl) P.rxl = p(x0 - 1, y, qk);
     if (c.hxh) {
-      P.rxh = p(x0 + c.cnt, y, qk);
-      P.rkx = Kx(x0 + c.cnt, y, qk);
+      P.rxh = p(x + V, y, qk);
+      P.rkx = Kx(x + V, y, qk);
     }
-    if (c.hyl) ldv<T, V>(p.at(x, y - 1, qk), n(), P.ryl);
+    if (c.hyl) ldv<T, V>(p.at(x, y - 1, qk), V, P.ryl);
     if (c.hyh) {
-      ldv<T, V>(p.at(x, y + 1, qk), n(), P.ryh);
-      ldv<T, V>(Ky.at(x, y + 1, qk), n(), P.rky);
+      ldv<T, V>(p.at(x, y + 1, qk), V, P.ryh);
+      ldv<T, V>(Ky.at(x, y + 1, qk), V, P.rky);
     }
   }
 
@@ -214,23 +251,23 @@ struct HeatColumn {
     const Plane &C = R[K % RING], &N = R[(K + 1) % RING];
     const int b = (z - z0) & 1, nn = n();
     if (act()) {
-      lds_st<T, V>(&L.sp[b][ly + 1][o], nn, C.p);
-      lds_st<T, V>(&L.skx[b][ly][o], nn, C.kx);
-      lds_st<T, V>(&L.sky[b][ly][V * lx], nn, C.ky);
+      lds_st<T, V>(&L.sp[b][ly + 1][o], V, C.p);
+      lds_st<T, V>(&L.skx[b][ly][o], V, C.kx);
+      lds_st<T, V>(&L.sky[b][ly][V * lx], V, C.ky);
       if (c.hxl) L.sp[b][ly + 1][V - 1] = C.rxl;
       if (c.hxh) {
-        L.sp[b][ly + 1][V + c.cnt] = C.rxh;
-        L.skx[b][ly][V + c.cnt] = C.rkx;
+        L.sp[b][ly + 1][o + V] = C.rxh;
+        L.skx[b][ly][o + V] = C.rkx;
       }
-      if (c.hyl) lds_st<T, V>(&L.sp[b][0][o], nn, C.ryl);
+      if (c.hyl) lds_st<T, V>(&L.sp[b][0][o], V, C.ryl);
       if (c.hyh) {
-        lds_st<T, V>(&L.sp[b][ly + 2][o], nn, C.ryh);
-        lds_st<T, V>(&L.sky[b][ly + 1][V * lx], nn, C.rky);
+        lds_st<T, V>(&L.sp[b][ly + 2][o], V, C.ryh);
+        lds_st<T, V>(&L.sky[b][ly + 1][V * lx], V, C.rky);
       }
-      // the slot takes plane z + PF + 1 (or, near the end, plane z1 again:
-      // the slot held plane z - 1, which is no longer needed)
-      load(min(z + PF + 1, z1), R[(K + PF + 1) % RING]);
     }
+    // the slot takes plane z + PF + 1 (or, near the end, plane z1 again:
+    // the slot held plane z - 1, which is no longer needed)
+    load(min(z + PF + 1, z1), R[(K + PF + 1) % RING]);
     __syncthreads();
     if (act()) {
       T pym[V], pyp[V], kyn[V], v[V];
@@ -241,8 +278,8 @@ struct HeatColumn {
 #pragma unroll
       for (int j = 0; j < V; j++) {
         const T pxm = j == 0 ? left : C.p[j == 0 ? 0 : j - 1];
-        const T pxp = j + 1 < nn ? C.p[j + 1 < V ? j + 1 : j] : L.sp[b][ly + 1][o + j + 1];
-        const T kxn = j + 1 < nn ? C.kx[j + 1 < V ? j + 1 : j] : L.skx[b][ly][o + j + 1];
+        const T pxp = j + 1 < V ? C.p[j + 1 < V ? j + 1 : j] : L.sp[b][ly + 1][o + V];
+        const T kxn = j + 1 < V ? C.kx[j + 1 < V ? j + 1 : j] : L.skx[b][ly][o + V];
         v[j] = ((T)1.0 + ry * (kyn[j] + C.ky[j]) + rx * (kxn + C.kx[j]) + rz * (N.kz[j] + C.kz[j])) * C.p[j] -
                ry * (kyn[j] * pyp[j] + C.ky[j] * pym[j]) - rx * (kxn * pxp + C.kx[j] * pxm) -
                rz * (N.kz[j] * N.p[j] + C.kz[j] * pm[j]);
@@ -279,11 +316,9 @@ struct HeatColumn {
     }
 #pragma unroll
     for (int j = 0; j < V; j++) pm[j] = (T)0;
-    if (act()) {
-      ldv<T, V>(p.at(x, y, z0 - 1), n(), pm);
+    ldv<T, V>(p.at(x, y, z0 - 1), V, pm);
 #pragma unroll
-      for (int i = 0; i < PF + 1; i++) load(min(z0 + i, z1), R[i]);
-    }
+    for (int i = 0; i < PF + 1; i++) load(min(z0 + i, z1), R[i]);
     int z = z0;
     for (; z + RING <= z1; z += RING) steps_all<0>(z);
     steps_tail<0>(z);
@@ -376,15 +411,15 @@ struct ChainColumn {
     ly = (int)threadIdx.y;
     cl = col_lane<V, WY>(x0, y0, R.x1, R.y1);
     if (FULL) cl.n = V;
-    x = x0 + V * lx;
-    y = y0 + ly;
+    x = x0 + V * (FULL ? lx : cl.lx);
+    y = y0 + (FULL ? ly : cl.ly);
     o = V + V * lx;
     in_xl = x0 - 1 >= R.x0;
-    in_xh = x0 + cl.cnt < R.x1;
+    in_xh = x + V < R.x1;
     in_yl = y - 1 >= R.y0;
     in_yh = y + 1 < R.y1;
     xl_r = in_xl ? x0 - 1 : x0;
-    xh_r = in_xh ? x0 + cl.cnt : x0 + cl.cnt - 1;
+    xh_r = in_xh ? x + V : x;
     yl_r = in_yl ? y - 1 : y;
     yh_r = in_yh ? y + 1 : y;
     acc = 0.0;
@@ -394,33 +429,38 @@ struct ChainColumn {
   // p_new of one value: the axpby inside R, p_old outside
   __device__ __forceinline__ double pnew(double po, double r, bool in) const { return in ? a * po + b * r : po; }
 
+  // p_new of the lane's points: p_old past the range end, which a last lane's
+  // vector may reach
+  __device__ __forceinline__ double pnew_at(int j, double po, double r, bool in) const {
+    return pnew(po, r, in && (FULL || j < cl.n));
+  }
+
   __device__ __forceinline__ void load(int q, ChainPlane<V> &Pl) const {
     const int qk = min(q, z1 - 1);
     const int qr = min(max(q, R.z0), R.z1 - 1);
-    const int nn = n();
-    ldv<double, V>(c.pold.at(x, y, q), nn, Pl.po);
-    ldv<double, V>(c.r.at(x, y, qr), nn, Pl.rr);
-    ldv<double, V, true>(c.Kz.at(x, y, q), nn, Pl.kz);
-    ldv<double, V, true>(c.Kx.at(x, y, qk), nn, Pl.kx);
-    ldv<double, V, true>(c.Ky.at(x, y, qk), nn, Pl.ky);
-    if (AXPY) ldv<double, V, true>(c.u.at(x, y, qk), nn, Pl.u);
+    ldv<double, V>(c.pold.at(x, y, q), V, Pl.po);
+    ldv<double, V>(c.r.at(x, y, qr), V, Pl.rr);
+    ldv<double, V, true>(c.Kz.at(x, y, q), V, Pl.kz);
+    ldv<double, V, true>(c.Kx.at(x, y, qk), V, Pl.kx);
+    ldv<double, V, true>(c.Ky.at(x, y, qk), V, Pl.ky);
+    if (AXPY) ldv<double, V, true>(c.u.at(x, y, qk), V, Pl.u);
     if (cl.hxl) {
       Pl.xl_po = c.pold(x0 - 1, y, qk);
       Pl.xl_r = c.r(xl_r, y, qk);
     }
     if (cl.hxh) {
-      Pl.xh_po = c.pold(x0 + cl.cnt, y, qk);
+      Pl.xh_po = c.pold(x + V, y, qk);
       Pl.xh_r = c.r(xh_r, y, qk);
-      Pl.xh_kx = c.Kx(x0 + cl.cnt, y, qk);
+      Pl.xh_kx = c.Kx(x + V, y, qk);
     }
     if (cl.hyl) {
-      ldv<double, V>(c.pold.at(x, y - 1, qk), nn, Pl.yl_po);
-      ldv<double, V>(c.r.at(x, yl_r, qk), nn, Pl.yl_r);
+      ldv<double, V>(c.pold.at(x, y - 1, qk), V, Pl.yl_po);
+      ldv<double, V>(c.r.at(x, yl_r, qk), V, Pl.yl_r);
     }
     if (cl.hyh) {
-      ldv<double, V>(c.pold.at(x, y + 1, qk), nn, Pl.yh_po);
-      ldv<double, V>(c.r.at(x, yh_r, qk), nn, Pl.yh_r);
-      ldv<double, V>(c.Ky.at(x, y + 1, qk), nn, Pl.yh_ky);
+      ldv<double, V>(c.pold.at(x, y + 1, qk), V, Pl.yh_po);
+      ldv<double, V>(c.r.at(x, yh_r, qk), V, Pl.yh_r);
+      ldv<double, V>(c.Ky.at(x, y + 1, qk), V, Pl.yh_ky);
     }
   }
 
@@ -430,33 +470,33 @@ struct ChainColumn {
     const int bb = (z - z0) & 1, nn = n();
     double pn[V];
     if (act()) {
-      lds_st<double, V>(&L.sp[bb][ly + 1][o], nn, pc);
-      lds_st<double, V>(&L.skx[bb][ly][o], nn, C.kx);
-      lds_st<double, V>(&L.sky[bb][ly][V * lx], nn, C.ky);
+      lds_st<double, V>(&L.sp[bb][ly + 1][o], V, pc);
+      lds_st<double, V>(&L.skx[bb][ly][o], V, C.kx);
+      lds_st<double, V>(&L.sky[bb][ly][V * lx], V, C.ky);
       if (cl.hxl) L.sp[bb][ly + 1][V - 1] = pnew(C.xl_po, C.xl_r, in_xl);
       if (cl.hxh) {
-        L.sp[bb][ly + 1][V + cl.cnt] = pnew(C.xh_po, C.xh_r, in_xh);
-        L.skx[bb][ly][V + cl.cnt] = C.xh_kx;
+        L.sp[bb][ly + 1][o + V] = pnew(C.xh_po, C.xh_r, in_xh);
+        L.skx[bb][ly][o + V] = C.xh_kx;
       }
       if (cl.hyl) {
         double t[V];
 #pragma unroll
         for (int j = 0; j < V; j++) t[j] = pnew(C.yl_po[j], C.yl_r[j], in_yl);
-        lds_st<double, V>(&L.sp[bb][0][o], nn, t);
+        lds_st<double, V>(&L.sp[bb][0][o], V, t);
       }
       if (cl.hyh) {
         double t[V];
 #pragma unroll
         for (int j = 0; j < V; j++) t[j] = pnew(C.yh_po[j], C.yh_r[j], in_yh);
-        lds_st<double, V>(&L.sp[bb][ly + 2][o], nn, t);
-        lds_st<double, V>(&L.sky[bb][ly + 1][V * lx], nn, C.yh_ky);
+        lds_st<double, V>(&L.sp[bb][ly + 2][o], V, t);
+        lds_st<double, V>(&L.sky[bb][ly + 1][V * lx], V, C.yh_ky);
       }
-      load(min(z + 2, z1), P[(K + 2) % RING]);
     }
+    load(min(z + 2, z1), P[(K + 2) % RING]);
     __syncthreads();
     const bool in_n = z + 1 < R.z1;
 #pragma unroll
-    for (int j = 0; j < V; j++) pn[j] = pnew(N.po[j], N.rr[j], in_n);
+    for (int j = 0; j < V; j++) pn[j] = pnew_at(j, N.po[j], N.rr[j], in_n);
     if (act()) {
       double pym[V], pyp[V], kyn[V], v[V], unew[V];
       lds_ld<double, V>(&L.sp[bb][ly][o], pym);
@@ -466,8 +506,8 @@ struct ChainColumn {
 #pragma unroll
       for (int j = 0; j < V; j++) {
         const double pxm = j == 0 ? left : pc[j == 0 ? 0 : j - 1];
-        const double pxp = j + 1 < nn ? pc[j + 1 < V ? j + 1 : j] : L.sp[bb][ly + 1][o + j + 1];
-        const double kxn = j + 1 < nn ? C.kx[j + 1 < V ? j + 1 : j] : L.skx[bb][ly][o + j + 1];
+        const double pxp = j + 1 < V ? pc[j + 1 < V ? j + 1 : j] : L.sp[bb][ly + 1][o + V];
+        const double kxn = j + 1 < V ? C.kx[j + 1 < V ? j + 1 : j] : L.skx[bb][ly][o + V];
         v[j] = (1.0 + ry * (kyn[j] + C.ky[j]) + rx * (kxn + C.kx[j]) + rz * (N.kz[j] + C.kz[j])) * pc[j] -
                ry * (kyn[j] * pyp[j] + C.ky[j] * pym[j]) - rx * (kxn * pxp + C.kx[j] * pxm) -
                rz * (N.kz[j] * pn[j] + C.kz[j] * pm[j]);
@@ -512,19 +552,17 @@ struct ChainColumn {
     }
 #pragma unroll
     for (int j = 0; j < V; j++) pm[j] = pc[j] = 0.0;
-    if (act()) {
-      // p_new of plane z0 - 1 (inside R when z0 > R.z0)
-      const int qm = z0 - 1;
-      double po[V], rv[V];
-      ldv<double, V>(c.pold.at(x, y, qm), n(), po);
-      ldv<double, V>(c.r.at(x, y, max(qm, R.z0)), n(), rv);
-      load(z0, P[0]);
-      load(min(z0 + 1, z1), P[1]);
+    // p_new of plane z0 - 1 (inside R when z0 > R.z0)
+    const int qm = z0 - 1;
+    double po[V], rv[V];
+    ldv<double, V>(c.pold.at(x, y, qm), V, po);
+    ldv<double, V>(c.r.at(x, y, max(qm, R.z0)), V, rv);
+    load(z0, P[0]);
+    load(min(z0 + 1, z1), P[1]);
 #pragma unroll
-      for (int j = 0; j < V; j++) {
-        pm[j] = pnew(po[j], rv[j], qm >= R.z0);
-        pc[j] = pnew(P[0].po[j], P[0].rr[j], true);
-      }
+    for (int j = 0; j < V; j++) {
+      pm[j] = pnew_at(j, po[j], rv[j], qm >= R.z0);
+      pc[j] = pnew_at(j, P[0].po[j], P[0].rr[j], true);
     }
     int z = z0;
     for (; z + RING <= z1; z += RING) steps_all<0>(z);
@@ -582,8 +620,8 @@ struct PoisColumn {
     ly = (int)threadIdx.y;
     c = col_lane<V, WY>(x0, y0, xe, ye);
     if (FULL) c.n = V;
-    x = x0 + V * lx;
-    y = y0 + ly;
+    x = x0 + V * (FULL ? lx : c.lx);
+    y = y0 + (FULL ? ly : c.ly);
     o = V + V * lx;
     acc = 0.0;
   }
@@ -592,11 +630,11 @@ struct PoisColumn {
 
   __device__ __forceinline__ void load(int q, PoisPlane<T, V> &P) const {
     const int qk = min(q, z1 - 1);
-    ldv<T, V>(p.at(x, y, q), n(), P.p);
+    ldv<T, V>(p.at(x, y, q), V, P.p);
     if (c.hxl) P.rxl = p(x0 - 1, y, qk);
-    if (c.hxh) P.rxh = p(x0 + c.cnt, y, qk);
-    if (c.hyl) ldv<T, V>(p.at(x, y - 1, qk), n(), P.ryl);
-    if (c.hyh) ldv<T, V>(p.at(x, y + 1, qk), n(), P.ryh);
+    if (c.hxh) P.rxh = p(x + V, y, qk);
+    if (c.hyl) ldv<T, V>(p.at(x, y - 1, qk), V, P.ryl);
+    if (c.hyh) ldv<T, V>(p.at(x, y + 1, qk), V, P.ryh);
   }
 
   template <int K>
@@ -604,13 +642,13 @@ struct PoisColumn {
     const PoisPlane<T, V> &C = R[K % RING], &N = R[(K + 1) % RING];
     const int b = (z - z0) & 1, nn = n();
     if (act()) {
-      lds_st<T, V>(&L.sp[b][ly + 1][o], nn, C.p);
+      lds_st<T, V>(&L.sp[b][ly + 1][o], V, C.p);
       if (c.hxl) L.sp[b][ly + 1][V - 1] = C.rxl;
-      if (c.hxh) L.sp[b][ly + 1][V + c.cnt] = C.rxh;
-      if (c.hyl) lds_st<T, V>(&L.sp[b][0][o], nn, C.ryl);
-      if (c.hyh) lds_st<T, V>(&L.sp[b][ly + 2][o], nn, C.ryh);
-      load(min(z + PF + 1, z1), R[(K + PF + 1) % RING]);
+      if (c.hxh) L.sp[b][ly + 1][o + V] = C.rxh;
+      if (c.hyl) lds_st<T, V>(&L.sp[b][0][o], V, C.ryl);
+      if (c.hyh) lds_st<T, V>(&L.sp[b][ly + 2][o], V, C.ryh);
     }
+    load(min(z + PF + 1, z1), R[(K + PF + 1) % RING]);
     __syncthreads();
     if (act()) {
       T pym[V], pyp[V], v[V];
@@ -620,7 +658,7 @@ struct PoisColumn {
 #pragma unroll
       for (int j = 0; j < V; j++) {
         const T pxm = j == 0 ? left : C.p[j == 0 ? 0 : j - 1];
-        const T pxp = j + 1 < nn ? C.p[j + 1 < V ? j + 1 : j] : L.sp[b][ly + 1][o + j + 1];
+        const T pxp = j + 1 < V ? C.p[j + 1 < V ? j + 1 : j] : L.sp[b][ly + 1][o + V];
         v[j] = (T)6.0 * C.p[j] - (pxm + pxp) - (pym[j] + pyp[j]) - (pm[j] + N.p[j]);
         if (j < nn) acc = acc + (double)v[j] * (double)C.p[j];
       }
@@ -655,11 +693,9 @@ struct PoisColumn {
     }
 #pragma unroll
     for (int j = 0; j < V; j++) pm[j] = (T)0;
-    if (act()) {
-      ldv<T, V>(p.at(x, y, z0 - 1), n(), pm);
+    ldv<T, V>(p.at(x, y, z0 - 1), V, pm);
 #pragma unroll
-      for (int i = 0; i < PF + 1; i++) load(min(z0 + i, z1), R[i]);
-    }
+    for (int i = 0; i < PF + 1; i++) load(min(z0 + i, z1), R[i]);
     int z = z0;
     for (; z + RING <= z1; z += RING) steps_all<0>(z);
     steps_tail<0>(z);
@@ -723,15 +759,15 @@ struct PoisChainColumn {
     ly = (int)threadIdx.y;
     cl = col_lane<V, WY>(x0, y0, R.x1, R.y1);
     if (FULL) cl.n = V;
-    x = x0 + V * lx;
-    y = y0 + ly;
+    x = x0 + V * (FULL ? lx : cl.lx);
+    y = y0 + (FULL ? ly : cl.ly);
     o = V + V * lx;
     in_xl = x0 - 1 >= R.x0;
-    in_xh = x0 + cl.cnt < R.x1;
+    in_xh = x + V < R.x1;
     in_yl = y - 1 >= R.y0;
     in_yh = y + 1 < R.y1;
     xl_r = in_xl ? x0 - 1 : x0;
-    xh_r = in_xh ? x0 + cl.cnt : x0 + cl.cnt - 1;
+    xh_r = in_xh ? x + V : x;
     yl_r = in_yl ? y - 1 : y;
     yh_r = in_yh ? y + 1 : y;
     acc = 0.0;
@@ -744,28 +780,33 @@ struct PoisChainColumn {
     else return a * rv + b * po;  // a = mi
   }
 
+  // p_new of the lane's points: p_old past the range end, which a last lane's
+  // vector may reach
+  __device__ __forceinline__ T pnew_at(int j, T po, T r, bool in) const {
+    return pnewv(po, r, in && (FULL || j < cl.n));
+  }
+
   __device__ __forceinline__ void load(int q, PoisChainPlane<T, V> &Pl) const {
     const int qk = min(q, z1 - 1);
     const int qr = min(max(q, R.z0), R.z1 - 1);
-    const int nn = n();
-    ldv<T, V>(pold.at(x, y, q), nn, Pl.po);
-    ldv<T, V>(r.at(x, y, qr), nn, Pl.rr);
-    if (AXPY) ldv<T, V, true>(u.at(x, y, qk), nn, Pl.u);
+    ldv<T, V>(pold.at(x, y, q), V, Pl.po);
+    ldv<T, V>(r.at(x, y, qr), V, Pl.rr);
+    if (AXPY) ldv<T, V, true>(u.at(x, y, qk), V, Pl.u);
     if (cl.hxl) {
       Pl.xl_po = pold(x0 - 1, y, qk);
       Pl.xl_r = r(xl_r, y, qk);
     }
     if (cl.hxh) {
-      Pl.xh_po = pold(x0 + cl.cnt, y, qk);
+      Pl.xh_po = pold(x + V, y, qk);
       Pl.xh_r = r(xh_r, y, qk);
     }
     if (cl.hyl) {
-      ldv<T, V>(pold.at(x, y - 1, qk), nn, Pl.yl_po);
-      ldv<T, V>(r.at(x, yl_r, qk), nn, Pl.yl_r);
+      ldv<T, V>(pold.at(x, y - 1, qk), V, Pl.yl_po);
+      ldv<T, V>(r.at(x, yl_r, qk), V, Pl.yl_r);
     }
     if (cl.hyh) {
-      ldv<T, V>(pold.at(x, y + 1, qk), nn, Pl.yh_po);
-      ldv<T, V>(r.at(x, yh_r, qk), nn, Pl.yh_r);
+      ldv<T, V>(pold.at(x, y + 1, qk), V, Pl.yh_po);
+      ldv<T, V>(r.at(x, yh_r, qk), V, Pl.yh_r);
     }
   }
 
@@ -775,27 +816,27 @@ struct PoisChainColumn {
     const int bb = (z - z0) & 1, nn = n();
     T pn[V];
     if (act()) {
-      lds_st<T, V>(&L.sp[bb][ly + 1][o], nn, pc);
+      lds_st<T, V>(&L.sp[bb][ly + 1][o], V, pc);
       if (cl.hxl) L.sp[bb][ly + 1][V - 1] = pnewv(C.xl_po, C.xl_r, in_xl);
-      if (cl.hxh) L.sp[bb][ly + 1][V + cl.cnt] = pnewv(C.xh_po, C.xh_r, in_xh);
+      if (cl.hxh) L.sp[bb][ly + 1][o + V] = pnewv(C.xh_po, C.xh_r, in_xh);
       if (cl.hyl) {
         T t[V];
 #pragma unroll
         for (int j = 0; j < V; j++) t[j] = pnewv(C.yl_po[j], C.yl_r[j], in_yl);
-        lds_st<T, V>(&L.sp[bb][0][o], nn, t);
+        lds_st<T, V>(&L.sp[bb][0][o], V, t);
       }
       if (cl.hyh) {
         T t[V];
 #pragma unroll
         for (int j = 0; j < V; j++) t[j] = pnewv(C.yh_po[j], C.yh_r[j], in_yh);
-        lds_st<T, V>(&L.sp[bb][ly + 2][o], nn, t);
+        lds_st<T, V>(&L.sp[bb][ly + 2][o], V, t);
       }
-      load(min(z + 2, z1), P[(K + 2) % RING]);
     }
+    load(min(z + 2, z1), P[(K + 2) % RING]);
     __syncthreads();
     const bool in_n = z + 1 < R.z1;
 #pragma unroll
-    for (int j = 0; j < V; j++) pn[j] = pnewv(N.po[j], N.rr[j], in_n);
+    for (int j = 0; j < V; j++) pn[j] = pnew_at(j, N.po[j], N.rr[j], in_n);
     if (act()) {
       T pym[V], pyp[V], v[V], unew[V];
       lds_ld<T, V>(&L.sp[bb][ly][o], pym);
@@ -804,7 +845,7 @@ struct PoisChainColumn {
 #pragma unroll
       for (int j = 0; j < V; j++) {
         const T pxm = j == 0 ? left : pc[j == 0 ? 0 : j - 1];
-        const T pxp = j + 1 < nn ? pc[j + 1 < V ? j + 1 : j] : L.sp[bb][ly + 1][o + j + 1];
+        const T pxp = j + 1 < V ? pc[j + 1 < V ? j + 1 : j] : L.sp[bb][ly + 1][o + V];
         v[j] = (T)6.0 * pc[j] - (pxm + pxp) - (pym[j] + pyp[j]) - (pm[j] + pn[j]);
         unew[j] = C.u[j] + alpha_u * C.po[j];
         if (j < nn) acc = acc + (double)v[j] * (double)pc[j];
@@ -846,18 +887,16 @@ struct PoisChainColumn {
     }
 #pragma unroll
     for (int j = 0; j < V; j++) pm[j] = pc[j] = (T)0;
-    if (act()) {
-      const int qm = z0 - 1;
-      T po[V], rv[V];
-      ldv<T, V>(pold.at(x, y, qm), n(), po);
-      ldv<T, V>(r.at(x, y, max(qm, R.z0)), n(), rv);
-      load(z0, P[0]);
-      load(min(z0 + 1, z1), P[1]);
+    const int qm = z0 - 1;
+    T po[V], rv[V];
+    ldv<T, V>(pold.at(x, y, qm), V, po);
+    ldv<T, V>(r.at(x, y, max(qm, R.z0)), V, rv);
+    load(z0, P[0]);
+    load(min(z0 + 1, z1), P[1]);
 #pragma unroll
-      for (int j = 0; j < V; j++) {
-        pm[j] = pnewv(po[j], rv[j], qm >= R.z0);
-        pc[j] = pnewv(P[0].po[j], P[0].rr[j], true);
-      }
+    for (int j = 0; j < V; j++) {
+      pm[j] = pnew_at(j, po[j], rv[j], qm >= R.z0);
+      pc[j] = pnew_at(j, P[0].po[j], P[0].rr[j], true);
     }
     int z = z0;
     for (; z + RING <= z1; z += RING) steps_all<0>(z);

@@ -199,7 +199,7 @@ int pois_chain_rule_t(std::vector<LoopRec> &run, size_t at) {
   if (U && !vec16_ok(U, R.x0)) ax = nullptr, U = nullptr;
   if (!use_vec() || cw.ctl.slot == nullptr) return 0;
   constexpr int V = 16 / (int)sizeof(T);
-  const ColGrid g = heat_column_grid(R, V * kWave, kHeatRows);
+  const ColGrid g = column_grid(R, V * kWave, kHeatRows);
   ensure_partials((size_t)g.blocks() * 8);
   PoisChainPtrs<T> c;
   DatView pv = view_of(P);

@@ -258,7 +258,7 @@ LoopRec make_heat3_loop(const char *name, const ops_arg *args, int nargs, const 
   if (INIT) vec = vec && vec16_ok(rr.dat, r.x0);
   ColGrid g;
   if (vec) {
-    g = heat_column_grid(r, 2 * kWave, kHeatRows);
+    g = INIT ? column_grid(r, 2 * kWave, kHeatRows) : heat_column_grid(r, 2 * kWave, kHeatRows);
   } else {
     g.chunk = heat_zchunk();
     g.gx = (unsigned)((r.x1 - r.x0 + kWave - 1) / kWave);
@@ -367,7 +367,7 @@ LoopRec make_poisson3_loop(const char *name, const ops_arg *args, int nargs, con
     return rec;
   }
   constexpr int V = 16 / (int)sizeof(T);
-  const ColGrid g = heat_column_grid(r, kWave * V, kHeatRows);
+  const ColGrid g = column_grid(r, kWave * V, kHeatRows);
   const RedCtl ctl = red_prepare(*red, 1, DT_F64, g.blocks());
   rec.ctl = ctl;
   rec.launch = [=](hipStream_t s) {
@@ -480,7 +480,7 @@ LoopRec make_stencil27_loop(const char *name, const ops_arg *args, int nargs, co
     rec.launch = [](hipStream_t) {};
     return rec;
   }
-  const ColGrid g = heat_column_grid(r, 2 * kWave, kHeatRows);
+  const ColGrid g = column_grid(r, 2 * kWave, kHeatRows);
   rec.launch = [=](hipStream_t s) {
     hipLaunchKernelGGL(k_stencil27_march, dim3(g.gx, g.gy, g.gz), dim3(kWave, kHeatRows), 0, s,
                        ptr_of<double>(out.dat), ptr_of<const double>(u.dat), r, g.chunk);

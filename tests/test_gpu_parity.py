@@ -780,3 +780,28 @@ def test_preproc_edges_and_remainders(gpu_ops, n):
         assert np.array_equal(ops.ops_dat_fetch_data(D[k]), np.where(inner, v, 1.0 if k[0] == "b" else 0.0)), k
     for q in D.values():
         ops.ops_free_dat(q)
+
+
+@pytest.mark.parametrize("n", [(130, 9, 5), (127, 8, 3), (129, 17, 66), (197, 15, 13), (254, 7, 131), (300, 33, 9),
+                               (2, 3, 70), (66, 1 + 8, 65)])
+def test_heat_column_tiles_and_chunks(gpu_ops, apps, n):
+    """Tiles that end inside a lane, a wave or a workgroup, and chunk lengths
+    from one plane to several chunks: the first CG iterations against the
+    oracle (fields' sums within 1e-12), at every fusion level the same bits."""
+    nx, ny, nz = n
+    K, rhs = O.heat_inputs(77, 3, nx, ny, nz)
+    ref = O.heat_cg(3, nx, ny, nz, K, rhs, max_iters=4, nthreads=NT)
+    got = []
+    for level in (0, 1, 2):
+        gpu_ops.ops_mi_set_fusion(level)
+        h = apps.Heat(3, nx, ny, nz, K_ext=K, rhs=rhs)
+        _, hist = h.iterate(4, history=True)
+        got.append((hist["pw"], hist["rrn"], h.u()))
+        h.close()
+    gpu_ops.ops_mi_set_fusion(2)
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            assert np.array_equal(a, b)
+    pw, rrn, u = got[0]
+    assert np.max(np.abs(rrn - ref["rrn"][1:]) / ref["rrn"][1:]) <= 1e-12
+    assert np.max(np.abs(u - ref["u"])) <= 1e-12 * np.max(np.abs(ref["u"]))
