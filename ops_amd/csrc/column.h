@@ -588,10 +588,11 @@ struct PoisLdsV {
 
 // one plane of a Poisson column as a lane loads it: its V points of p and
 // the rims it owns
-template <class T, int V>
+template <class T, int V, bool RES = false>
 struct PoisPlane {
   T p[V], ryl[V], ryh[V];
   T rxl, rxh;
+  T f[RES ? V : 1];
 };
 
 // w = 6p - (p(-1,0,0) + p(1,0,0)) - (p(0,-1,0) + p(0,1,0)) - (p(0,0,-1) +
@@ -599,23 +600,25 @@ struct PoisPlane {
 // (double) w (double) p.  Same structure as HeatColumn: PF planes of loads
 // ahead in an unrolled register ring, the same loads every step (the rims of
 // plane z1, never used, come from plane z1 - 1), and a branch-free form for
-// tiles inside the range.
-template <class T, int V, bool NT, int WY, int PF, bool FULL>
+// tiles inside the range.  RES: w = f - A p instead, and the sum of its
+// squares.
+template <class T, int V, bool NT, int WY, int PF, bool FULL, bool RES>
 struct PoisColumn {
   static constexpr int RING = PF + 2;
   PoisLdsV<T, V, WY> &L;
   const Ptr<T> &w;
-  const Ptr<const T> &p;
+  const Ptr<const T> &p, &f;
   int x0, z0, z1;
   ColLane c;
   int x, y, o, lx, ly;
   double acc;
   T pm[V];
-  PoisPlane<T, V> R[RING];
+  using Plane = PoisPlane<T, V, RES>;
+  Plane R[RING];
 
-  __device__ __forceinline__ PoisColumn(PoisLdsV<T, V, WY> &L_, const Ptr<T> &w_, const Ptr<const T> &p_, int x0_,
-                                        int y0, int xe, int ye, int z0_, int z1_)
-      : L(L_), w(w_), p(p_), x0(x0_), z0(z0_), z1(z1_) {
+  __device__ __forceinline__ PoisColumn(PoisLdsV<T, V, WY> &L_, const Ptr<T> &w_, const Ptr<const T> &p_,
+                                        const Ptr<const T> &f_, int x0_, int y0, int xe, int ye, int z0_, int z1_)
+      : L(L_), w(w_), p(p_), f(f_), x0(x0_), z0(z0_), z1(z1_) {
     lx = (int)threadIdx.x;
     ly = (int)threadIdx.y;
     c = col_lane<V, WY>(x0, y0, xe, ye);
@@ -628,18 +631,19 @@ struct PoisColumn {
   __device__ __forceinline__ int n() const { return FULL ? V : c.n; }
   __device__ __forceinline__ bool act() const { return FULL || c.n > 0; }
 
-  __device__ __forceinline__ void load(int q, PoisPlane<T, V> &P) const {
+  __device__ __forceinline__ void load(int q, Plane &P) const {
     const int qk = min(q, z1 - 1);
     ldv<T, V>(p.at(x, y, q), V, P.p);
     if (c.hxl) P.rxl = p(x0 - 1, y, qk);
     if (c.hxh) P.rxh = p(x + V, y, qk);
     if (c.hyl) ldv<T, V>(p.at(x, y - 1, qk), V, P.ryl);
     if (c.hyh) ldv<T, V>(p.at(x, y + 1, qk), V, P.ryh);
+    if constexpr (RES) ldv<T, V, true>(f.at(x, y, qk), V, P.f);
   }
 
   template <int K>
   __device__ __forceinline__ void step(int z) {
-    const PoisPlane<T, V> &C = R[K % RING], &N = R[(K + 1) % RING];
+    const Plane &C = R[K % RING], &N = R[(K + 1) % RING];
     const int b = (z - z0) & 1, nn = n();
     if (act()) {
       lds_st<T, V>(&L.sp[b][ly + 1][o], V, C.p);
@@ -660,7 +664,12 @@ struct PoisColumn {
         const T pxm = j == 0 ? left : C.p[j == 0 ? 0 : j - 1];
         const T pxp = j + 1 < V ? C.p[j + 1 < V ? j + 1 : j] : L.sp[b][ly + 1][o + V];
         v[j] = (T)6.0 * C.p[j] - (pxm + pxp) - (pym[j] + pyp[j]) - (pm[j] + N.p[j]);
-        if (j < nn) acc = acc + (double)v[j] * (double)C.p[j];
+        if constexpr (RES) {
+          v[j] = C.f[j] - v[j];
+          if (j < nn) acc = acc + (double)v[j] * (double)v[j];
+        } else {
+          if (j < nn) acc = acc + (double)v[j] * (double)C.p[j];
+        }
       }
       stv<T, V, NT>(w.at(x, y, z), nn, v);
     }
@@ -688,7 +697,7 @@ struct PoisColumn {
 #pragma unroll
     for (int i = 0; i < RING; i++) {
 #pragma unroll
-      for (int j = 0; j < V; j++) R[i].p[j] = R[i].ryl[j] = R[i].ryh[j] = (T)0;
+      for (int j = 0; j < V; j++) R[i].p[j] = R[i].ryl[j] = R[i].ryh[j] = R[i].f[RES ? j : 0] = (T)0;
       R[i].rxl = R[i].rxh = (T)0;
     }
 #pragma unroll
@@ -703,12 +712,13 @@ struct PoisColumn {
   }
 };
 
-template <class T, int V, bool NT, int WY = kWavesPerBlock, int PF = 1>
+template <class T, int V, bool NT, int WY = kWavesPerBlock, int PF = 1, bool RES = false>
 __device__ __forceinline__ double poisson3_column_v(PoisLdsV<T, V, WY> &L, const Ptr<T> &w, const Ptr<const T> &p,
-                                                    int x0, int y0, int xe, int ye, int z0, int z1) {
+                                                    const Ptr<const T> &f, int x0, int y0, int xe, int ye, int z0,
+                                                    int z1) {
   if (x0 + kWave * V <= xe && y0 + WY <= ye)
-    return PoisColumn<T, V, NT, WY, PF, true>(L, w, p, x0, y0, xe, ye, z0, z1).run();
-  return PoisColumn<T, V, NT, WY, PF, false>(L, w, p, x0, y0, xe, ye, z0, z1).run();
+    return PoisColumn<T, V, NT, WY, PF, true, RES>(L, w, p, f, x0, y0, xe, ye, z0, z1).run();
+  return PoisColumn<T, V, NT, WY, PF, false, RES>(L, w, p, f, x0, y0, xe, ye, z0, z1).run();
 }
 
 // ------------------------------------------------------------ fused Poisson CG chains

@@ -347,9 +347,9 @@ __global__ __launch_bounds__(kWave * kHeatRows) void k_poisson3_march(Ptr<T> w, 
   __shared__ PoisLdsV<T, V, kHeatRows> lds;
   const TileId t = tile_id();
   const int z0 = rg.z0 + (int)t.z * chunk;
-  double acc[1] = {poisson3_column_v<T, V, true, kHeatRows, kPoisPF>(lds, w, p, rg.x0 + (int)t.x * kWave * V,
-                                                                     rg.y0 + (int)t.y * kHeatRows, rg.x1, rg.y1, z0,
-                                                                     min(z0 + chunk, rg.z1))};
+  double acc[1] = {poisson3_column_v<T, V, true, kHeatRows, kPoisPF>(
+      lds, w, p, Ptr<const T>{nullptr, 0, 0}, rg.x0 + (int)t.x * kWave * V, rg.y0 + (int)t.y * kHeatRows, rg.x1, rg.y1,
+      z0, min(z0 + chunk, rg.z1))};
   reduce_block_store<double, OPS_INC, 1>(acc, ctl);
 }
 

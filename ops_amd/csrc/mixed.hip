@@ -18,6 +18,7 @@
 // preconditioned residual z = Mi rr is recomputed where it is needed instead
 // of being stored: 44 bytes per point per inner iteration (4 + 4, 8 + 8 + 4 +
 // 4, 8 + 4) against 88 for an FP64 CG iteration.
+#include "column.h"
 #include "engine.h"
 
 using namespace opsmi;
@@ -43,6 +44,42 @@ struct PoissonRes {
     s[0] = s[0] + v * v;
   }
 };
+
+// 3D form as an LDS z-column (poisson3_column_v), bounded by its 24 bytes a
+// point: each plane of x is loaded once instead of seven times from the
+// caches.  400 x 384 x 390: 444 us (3.2 TB/s) on the generic engine,
+// 317 us (4.5 TB/s) now.
+__global__ __launch_bounds__(kWave * kHeatRows) void k_poisson3_residual(Ptr<double> r, Ptr<const double> f,
+                                                                         Ptr<const double> x, Range3 rg, int chunk,
+                                                                         RedCtl ctl) {
+  constexpr int V = 2;
+  __shared__ PoisLdsV<double, V, kHeatRows> lds;
+  const TileId t = tile_id();
+  const int z0 = rg.z0 + (int)t.z * chunk;
+  double acc[1] = {poisson3_column_v<double, V, true, kHeatRows, 2, true>(
+      lds, r, x, f, rg.x0 + (int)t.x * kWave * V, rg.y0 + (int)t.y * kHeatRows, rg.x1, rg.y1, z0,
+      min(z0 + chunk, rg.z1))};
+  reduce_block_store<double, OPS_INC, 1>(acc, ctl);
+}
+
+LoopRec make_residual3_loop(const char *name, const ops_arg *args, int nargs, const Range3 &rg, ops_dat r, ops_dat f,
+                            ops_dat x, const ops_arg *red) {
+  LoopRec rec;
+  rec.name = name ? name : "?";
+  rec.range = rg;
+  rec.bytes = transfer_bytes(args, nargs, rg);
+  deps_from_args(rec, args, nargs);
+  const ColGrid g = column_grid(rg, kWave * 2, kHeatRows);
+  const RedCtl ctl = red_prepare(*red, 1, DT_F64, g.blocks());
+  rec.ctl = ctl;
+  rec.launch = [=](hipStream_t s) {
+    const RedCtl c = with_host_fold(ctl, g.blocks(), 1, DT_F64);
+    hipLaunchKernelGGL(k_poisson3_residual, dim3(g.gx, g.gy, g.gz), dim3(kWave, kHeatRows), 0, s, ptr_of<double>(r),
+                       ptr_of<const double>(f), ptr_of<const double>(x), rg, g.chunk, c);
+    launch_red_finish<double, OPS_INC, 1>(c, g.blocks(), s);
+  };
+  return rec;
+}
 
 struct MpInit {
   using red_t = double;
@@ -230,7 +267,12 @@ void ops_par_loop_poisson_residual_kernel(const char *name, ops_block block, int
                          {dat_w(DT_F64), dat_r(pts_point(), DT_F64), dat_r(dim == 3 ? pts_7pt() : pts_5pt(), DT_F64),
                           red_a(OPS_INC, DT_F64)},
                          nullptr);
-  if (dim == 2)
+  // the column needs 16-byte rows, and r apart from what its neighbours read
+  const bool col = dim == 3 && rg.npts() > 0 && use_vec() && r.dat != x.dat && r.dat != f.dat &&
+                   vec16_ok(r.dat, rg.x0) && vec16_ok(f.dat, rg.x0) && vec16_ok(x.dat, rg.x0);
+  if (col)
+    enqueue(make_residual3_loop(name, args, nargs, rg, r.dat, f.dat, x.dat, &rr));
+  else if (dim == 2)
     launch_loop(name, args, nargs, rg, [=] {
       return PoissonRes<2>{ptr_of<double>(r.dat), ptr_of<const double>(f.dat), ptr_of<const double>(x.dat)};
     }, &rr);

@@ -163,3 +163,59 @@ def test_mixed_solve_matches_oracle(gpu_ops, n):
     cg = O.poisson_cg(nd, nx, ny, nz, f, max_iters=5000, tol=1e-13, nthreads=8)
     err = np.max(np.abs(x - cg["x"])) / np.max(np.abs(cg["x"]))
     assert err <= 1e-8
+
+
+@pytest.mark.parametrize("n", [(2, 3, 4), (126, 8, 5), (129, 9, 3), (130, 17, 66), (258, 5, 9)])
+def test_residual_column_tile_edges(gpu_ops, n):
+    """the 3D residual's tiles of 128 x 8 points, their remainders and chunks"""
+    test_residual_kernel_matches_oracle(gpu_ops, n)
+
+
+@pytest.mark.parametrize("n", [(254, 9, 3), (257, 8, 5), (260, 17, 66), (400, 5, 9), (30, 3, 70)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_poisson_columns_tile_edges(gpu_ops, n, dtype):
+    """sweep and chain columns at the remainders of their 128- or 256-point
+    tiles: three CG-like steps at fusion levels 0 and 2 give the same bits,
+    and the sweep is the operator's (numpy, the kernel's order)"""
+    ops = gpu_ops
+    f64 = dtype is np.float64
+    ty = "double" if f64 else "float"
+    blk, s0, rg = _setup(ops, n)
+    sp = ops.ops_decl_stencil(3, 7, O_pts(3), "sp")
+    rng = np.random.RandomState(4)
+    R, RW, W = ops.OPS_READ, ops.OPS_RW, ops.OPS_WRITE
+    init = {k: rng.rand(*n[::-1]).astype(dtype) for k in "urp"}
+    out = []
+    for level in (0, 2):
+        ops.ops_mi_set_fusion(level)
+        D = {k: ops.ops_decl_dat(blk, list(n), dtype=dtype, name=k) for k in "urpw"}
+        for k, v in init.items():
+            ops.ops_dat_set_data(D[k], v)
+        red = ops.ops_decl_reduction_handle(8, "double", "pw")
+        A = lambda k, s, acc: ops.ops_arg_dat(D[k], 1, s, ty, acc)
+        sums = []
+        for it in range(3):
+            g = lambda v: ops.ops_arg_gbl(v, 1, ty)
+            if f64:
+                ops.ops_par_loop("tea_leaf_axpy_kernel", "axpy", blk, 3, rg, A("u", s0, ops.OPS_INC), A("p", s0, R), g(0.5))
+                ops.ops_par_loop("tea_leaf_axpby_kernel", "axpby", blk, 3, rg, A("p", s0, RW), A("r", s0, R), g(0.25),
+                                 g(1.0))
+            else:
+                ops.ops_par_loop("mp_e_update_kernel", "e", blk, 3, rg, A("u", s0, RW), A("p", s0, R), g(0.5))
+                ops.ops_par_loop("mp_p_kernel", "p", blk, 3, rg, A("p", s0, RW), A("r", s0, R), g(1.0), g(0.25))
+            ops.ops_par_loop("poisson_calc_w_reduce_kernel", "w", blk, 3, rg, A("w", s0, W), A("p", sp, R),
+                             ops.ops_arg_reduce(red, 1, "double", ops.OPS_INC))
+            sums.append(float(ops.ops_reduction_result(red)))
+        out.append([np.array(sums)] + [ops.ops_dat_fetch_data(D[k]) for k in "upw"])
+        for d in D.values():
+            ops.ops_free_dat(d)
+    ops.ops_mi_set_fusion(2)
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    _, _, p, w = out[0]
+    e = np.zeros([v + 2 for v in p.shape], dtype)
+    e[1:-1, 1:-1, 1:-1] = p
+    c = slice(1, -1)
+    ref = dtype(6) * p - (e[c, c, :-2] + e[c, c, 2:]) - (e[c, :-2, c] + e[c, 2:, c]) - (e[:-2, c, c] + e[2:, c, c])
+    assert np.array_equal(w, ref)
+    assert abs(out[0][0][-1] - np.sum(w.astype(np.float64) * p)) <= 1e-12 * np.sum(np.abs(w.astype(np.float64) * p))
