@@ -244,10 +244,19 @@ int pois_chain_rule_level2(std::vector<LoopRec> &run, size_t at, hipStream_t s) 
 // where A' is A after the copy (Anew_old inside R, A's own values outside).
 // Anew' goes to Anew's spare buffer (neighbouring waves still read
 // Anew_old), which then becomes Anew's buffer.  24 bytes per point instead of
-// 16 + 16, and one launch.  Each wave marches kJacRows rows of a (64 V)-wide
+// 16 + 16, and one launch.  Each wave marches `rows` rows of a (64 V)-wide
 // strip keeping three rows in registers; x neighbours come from the adjacent
 // lanes (shuffles) and, at the strip ends, one scalar load.
-constexpr int kJacRows = 16;
+//
+// Bounded by HBM on large grids and by the march's latency (0.6 us a row) on
+// small ones: kJacRows rows a wave, halved while the grid has fewer than
+// kJacWaves waves, and to single rows below kJacFew.  Timed with events:
+// 96 x 70 13.2 us with 16 rows (5 waves), 5.9 us with one; 1500^2 20.9 with 16,
+// 14.1 with 4; at 2048^2 16 rows 18.3-19.1 us, 8 rows 19.1, 4 rows 18.8, 2 rows
+// 18.2, 1 row 25.2.  A is stored past the caches: the next pass reads it at
+// the halo only, and Anew, which it reads throughout, keeps the room (4094^2
+// 89 us with plain stores, 70 us so; Anew stored so too: 86 us).
+constexpr int kJacRows = 16, kJacWaves = 4096, kJacFew = 1024;
 
 template <class T>
 struct JacPtrs {
@@ -255,33 +264,36 @@ struct JacPtrs {
   Ptr<const T> An;
 };
 
-// FULL: every tile is 64 V points wide inside the range (every lane has V
-// points): the element counts are literals, the edge values are loaded by
-// every lane (one broadcast address) and kept by the edge lane, so a row has
-// no lane-divergent branches (a branch join makes the compiler wait for
-// every load in flight), and each row is loaded one row ahead of its use
+// FULL: every tile is 64 V points wide inside the range.  Otherwise a lane
+// past the range's end loads the last lane's vectors, and the last lane whole
+// ones (see column.h), so that no form has lane-divergent loads (a branch join
+// makes the compiler wait for every load in flight).  The edge values are loaded by every lane (one
+// broadcast address) and kept by the edge lane, and each row is loaded one
+// row ahead of its use.
 template <class T, int V, bool FULL>
-__global__ __launch_bounds__(kWave * kWavesPerBlock) void k_jacobi_chain(JacPtrs<T> c, Range3 R, RedCtl ctl) {
+__global__ __launch_bounds__(kWave * kWavesPerBlock) void k_jacobi_chain(JacPtrs<T> c, Range3 R, int rows,
+                                                                         RedCtl ctl) {
   T err[1] = {RedOp<T, OPS_MAX>::identity()};
   const int lx = (int)threadIdx.x, wv = (int)threadIdx.y;
   const TileId t = tile_id();
   const int x0 = R.x0 + (int)t.x * kWave * V;
-  const int ya = R.y0 + ((int)t.y * kWavesPerBlock + wv) * kJacRows;
-  const int yb = min(ya + kJacRows, R.y1);
+  const int ya = R.y0 + ((int)t.y * kWavesPerBlock + wv) * rows;
+  const int yb = min(ya + rows, R.y1);
   const int z = R.z0;
   const int cnt = FULL ? kWave * V : min(kWave * V, R.x1 - x0);
-  const int x = x0 + V * lx;
+  const int last = (cnt - 1) / V;
   const int n = FULL ? V : max(0, min(V, cnt - V * lx));
-  const bool hxh = lx == (cnt - 1) / V;
+  const int x = x0 + V * (FULL ? lx : min(lx, last));
+  const bool hxh = lx == last;
   const bool in_xl = x0 - 1 >= R.x0, in_xh = x0 + cnt < R.x1;
   auto row = [&](int yy, T (&v)[V]) {
     const bool in = yy >= R.y0 && yy < R.y1;
-    ldv<T, V>(in ? c.An.at(x, yy, z) : (const T *)c.A.at(x, yy, z), n, v);
+    ldv<T, V>(in ? c.An.at(x, yy, z) : (const T *)c.A.at(x, yy, z), V, v);
   };
   auto edge = [&](int xx, int yy, bool inx) -> T {
     return inx && yy >= R.y0 && yy < R.y1 ? c.An(xx, yy, z) : c.A(xx, yy, z);
   };
-  if (FULL && ya < yb) {
+  if (ya < yb) {
     // rows y + 1 and y + 2 are in registers while row y is computed (the
     // load of row y + 2 is issued one row ahead; rows past yb read row yb,
     // a row of the range or its halo)
@@ -302,50 +314,18 @@ __global__ __launch_bounds__(kWave * kWavesPerBlock) void k_jacobi_chain(JacPtrs
 #pragma unroll
       for (int j = 0; j < V; j++) {
         const T xm = j > 0 ? cur[j > 0 ? j - 1 : 0] : (lx == 0 ? cl : fromleft);
-        const T xp = j + 1 < V ? cur[j + 1 < V ? j + 1 : j] : (hxh ? cr : fromright);
+        T xp = j + 1 < V ? cur[j + 1 < V ? j + 1 : j] : fromright;
+        if (hxh && j + 1 == n) xp = cr;  // past the range's end A keeps its own values
         v[j] = (T)0.25f * (xp + xm + up[j] + dn[j]);
-        err[0] = RedOp<T, OPS_MAX>::combine(err[0], fabs(v[j] - cur[j]));
+        if (FULL || j < n) err[0] = RedOp<T, OPS_MAX>::combine(err[0], fabs(v[j] - cur[j]));
       }
-      stv<T, V, false>(c.A.at(x, y, z), V, cur);
-      stv<T, V, false>(c.out.at(x, y, z), V, v);
+      stv<T, V, true>(c.A.at(x, y, z), n, cur);
+      stv<T, V, false>(c.out.at(x, y, z), n, v);
 #pragma unroll
       for (int j = 0; j < V; j++) {
         up[j] = cur[j];
         cur[j] = dn[j];
         dn[j] = dn2[j];
-      }
-      cl = ncl;
-      cr = ncr;
-    }
-  } else if (ya < yb) {
-    T up[V], cur[V], dn[V];
-    row(ya - 1, up);
-    row(ya, cur);
-    T cl = lx == 0 ? edge(x0 - 1, ya, in_xl) : (T)0, cr = hxh ? edge(x0 + cnt, ya, in_xh) : (T)0;
-    for (int y = ya; y < yb; y++) {
-      row(y + 1, dn);
-      T ncl = 0, ncr = 0;
-      if (y + 1 < yb) {
-        if (lx == 0) ncl = edge(x0 - 1, y + 1, in_xl);
-        if (hxh) ncr = edge(x0 + cnt, y + 1, in_xh);
-      }
-      const T fromleft = __shfl_up(cur[V - 1], 1, kWave), fromright = __shfl_down(cur[0], 1, kWave);
-      T v[V];
-#pragma unroll
-      for (int j = 0; j < V; j++) {
-        const T xm = j > 0 ? cur[j > 0 ? j - 1 : 0] : (lx == 0 ? cl : fromleft);
-        const T xp = j + 1 < n ? cur[j + 1 < V ? j + 1 : j] : (hxh ? cr : fromright);
-        v[j] = (T)0.25f * (xp + xm + up[j] + dn[j]);
-        if (j < n) err[0] = RedOp<T, OPS_MAX>::combine(err[0], fabs(v[j] - cur[j]));
-      }
-      if (n > 0) {
-        stv<T, V, false>(c.A.at(x, y, z), n, cur);
-        stv<T, V, false>(c.out.at(x, y, z), n, v);
-      }
-#pragma unroll
-      for (int j = 0; j < V; j++) {
-        up[j] = cur[j];
-        cur[j] = dn[j];
       }
       cl = ncl;
       cr = ncr;
@@ -358,8 +338,11 @@ template <class T>
 void launch_jacobi_chain(const LoopRec &cp, const LoopRec &jac, const Range3 &R) {
   constexpr int V = 16 / (int)sizeof(T);
   ops_dat A = jac.d[0], An = jac.d[1];
-  const unsigned gx = (unsigned)((R.x1 - R.x0 + kWave * V - 1) / (kWave * V));
-  const unsigned gy = (unsigned)((R.y1 - R.y0 + kWavesPerBlock * kJacRows - 1) / (kWavesPerBlock * kJacRows));
+  const long nx = R.x1 - R.x0, ny = R.y1 - R.y0;
+  const unsigned gx = (unsigned)((nx + kWave * V - 1) / (kWave * V));
+  int rows = kJacRows;
+  while (rows > 1 && gx * ((ny + rows - 1) / rows) < (rows > 2 ? kJacWaves : kJacFew)) rows /= 2;
+  const unsigned gy = (unsigned)((ny + kWavesPerBlock * rows - 1) / (kWavesPerBlock * rows));
   ensure_partials((size_t)gx * gy * sizeof(T));
   JacPtrs<T> c;
   DatView v = view_of(An);
@@ -368,9 +351,8 @@ void launch_jacobi_chain(const LoopRec &cp, const LoopRec &jac, const Range3 &R)
   c.An = ptr_of<const T>(An);
   const RedCtl ctl = with_host_fold(jac.ctl, gx * gy, 1, sizeof(T) == 8 ? DT_F64 : DT_F32);
   run_loop("jacobi_chain(copy+apply_stencil)", cp.bytes + jac.bytes, [&](hipStream_t st) {
-    // every tile whole: the branch-free form
-    auto kern = (R.x1 - R.x0) % (kWave * V) == 0 ? k_jacobi_chain<T, V, true> : k_jacobi_chain<T, V, false>;
-    hipLaunchKernelGGL(kern, dim3(gx, gy, 1), dim3(kWave, kWavesPerBlock), 0, st, c, R, ctl);
+    auto kern = nx % (kWave * V) == 0 ? k_jacobi_chain<T, V, true> : k_jacobi_chain<T, V, false>;
+    hipLaunchKernelGGL(kern, dim3(gx, gy, 1), dim3(kWave, kWavesPerBlock), 0, st, c, R, rows, ctl);
     launch_red_finish<T, OPS_MAX, 1>(ctl, gx * gy, st);
   });
   swap_spare(An, R);

@@ -805,3 +805,16 @@ def test_heat_column_tiles_and_chunks(gpu_ops, apps, n):
     pw, rrn, u = got[0]
     assert np.max(np.abs(rrn - ref["rrn"][1:]) / ref["rrn"][1:]) <= 1e-12
     assert np.max(np.abs(u - ref["u"])) <= 1e-12 * np.max(np.abs(ref["u"]))
+
+
+@pytest.mark.parametrize("n", [(2, 2), (3, 70), (127, 5), (128, 9), (129, 17), (255, 1030), (257, 40), (1500, 260),
+                               (600, 2300)])
+def test_laplace_rows_and_strips(apps, n):
+    """strips that end inside a lane or a wave, and every number of rows a
+    wave takes (1 to 16): bit-exact, as averages and a maximum are"""
+    nx, ny = n
+    init = O.laplace_init(nx, ny, 0)
+    _, hist, A = apps.laplace2d(nx, ny, 7, 0, init)
+    A_ref, h_ref = O.laplace_run(init, 7)
+    assert np.array_equal(hist, h_ref)
+    assert np.array_equal(A, O.interior(A_ref))
