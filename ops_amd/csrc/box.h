@@ -21,6 +21,10 @@ struct Box {
 // array) holds the values
 void box_copy(Staging &st, hipStream_t s, Box b, char *buf, bool to_device);
 
+// dst = src outside the points of r, both whole arrays laid out as d's (one
+// array: not structure of arrays), on the library's stream
+void copy_outside(ops_dat d, char *dst, const char *src, const Range3 &r);
+
 // whether a caller's buffer is device memory (fetch and set take either kind)
 bool device_pointer(const void *p);
 

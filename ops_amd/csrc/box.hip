@@ -72,6 +72,27 @@ __global__ __launch_bounds__(256) void k_box(Box b, char *host, unsigned row, si
   }
 }
 
+// a whole array's rows outside [r0, r1) x [y0, y1) x [z0, z1) of raw units,
+// rows and planes: a wave per row and kSegment of its units, which copies all
+// of them or those left and right of the range
+constexpr unsigned kSegment = 1024;
+template <int U>
+__global__ __launch_bounds__(256) void k_outside(char *dst, const char *src, unsigned pitch, unsigned rows,
+                                                 unsigned total, unsigned r0, unsigned r1, unsigned y0, unsigned y1,
+                                                 unsigned z0, unsigned z1) {
+  typedef typename unit_of<U>::type T;
+  const unsigned row = blockIdx.x * 4 + threadIdx.x / 64, lane = threadIdx.x % 64;
+  if (row >= total) return;
+  const unsigned y = row % rows, z = row / rows;
+  const bool inside = y >= y0 && y < y1 && z >= z0 && z < z1;
+  const T *s = (const T *)src + (size_t)row * pitch;
+  T *d = (T *)dst + (size_t)row * pitch;
+  const unsigned lo = blockIdx.y * kSegment, hi = min(lo + kSegment, pitch);
+  if (inside && lo >= r0 && hi <= r1) return;
+  for (unsigned i = lo + lane; i < hi; i += 64)
+    if (!inside || i < r0 || i >= r1) d[i] = s[i];
+}
+
 template <int U>
 void launch(const Box &b, char *host, bool to_device, unsigned row, size_t col, unsigned n, hipStream_t s) {
   const dim3 g((n + 256u * kPerThread - 1) / (256u * kPerThread));
@@ -116,6 +137,39 @@ void Staging::ensure() {
     }
     if (!ev[q]) OPSMI_HIP(hipEventCreateWithFlags(&ev[q], hipEventDisableTiming));
   }
+}
+
+void copy_outside(ops_dat d, char *dst, const char *src, const Range3 &r) {
+  const int nd = d->block->dims;
+  const int lo[3] = {r.x0, r.y0, r.z0}, hi[3] = {r.x1, r.y1, r.z1};
+  unsigned a[3] = {0, 0, 0}, b[3] = {1, 1, 1};
+  for (int q = 0; q < nd; q++) {  // raw indexes
+    const int first = d->d_m[q] + d->base[q];
+    a[q] = (unsigned)std::min(std::max(lo[q] - first, 0), d->size[q]);
+    b[q] = (unsigned)std::min(std::max(hi[q] - first, 0), d->size[q]);
+  }
+  const size_t total = (size_t)d->size[1] * d->size[2];
+  int U = 16;
+  const size_t es = d->elem_size;
+  // units that whole points and the allocation's start are multiples of (the
+  // range's ends fall on points)
+  while (es % U || (uintptr_t)src % U || (uintptr_t)dst % U) U /= 2;
+  const size_t per = es / U, pitch = d->size[0] * per;
+  if (total >> 31 || pitch / kSegment > 65000) {
+    OPSMI_HIP(hipMemcpyAsync(dst, src, d->mem, hipMemcpyDeviceToDevice, inst().stream));
+    return;
+  }
+  const dim3 g((unsigned)((total + 3) / 4), (unsigned)((pitch + kSegment - 1) / kSegment));
+  auto go = [&](auto k) {
+    hipLaunchKernelGGL(k, g, dim3(256), 0, inst().stream, dst, src, (unsigned)pitch, (unsigned)d->size[1],
+                       (unsigned)total, (unsigned)(a[0] * per), (unsigned)(b[0] * per), a[1], b[1], a[2], b[2]);
+  };
+  if (U == 16) go(k_outside<16>);
+  else if (U == 8) go(k_outside<8>);
+  else if (U == 4) go(k_outside<4>);
+  else if (U == 2) go(k_outside<2>);
+  else go(k_outside<1>);
+  OPSMI_HIP(hipGetLastError());
 }
 
 void box_copy(Staging &st, hipStream_t s, Box b, char *buf, bool to_device) {

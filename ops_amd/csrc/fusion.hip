@@ -78,7 +78,7 @@ int cg_chain_rule(std::vector<LoopRec> &run, size_t at, hipStream_t s) {
   ensure_partials((size_t)g.blocks() * 8);
   ChainPtrs c;
   DatView pv = view_of(P);
-  c.pnew = Ptr<double>{(double *)spare_base(P, R), pv.sy, pv.sz};
+  c.pnew = Ptr<double>{(double *)spare_base(P, R, true), pv.sy, pv.sz};
   c.pold = ptr_of<const double>(P);
   c.r = ptr_of<const double>(Rr);
   c.w = ptr_of<double>(W);
@@ -203,7 +203,7 @@ int pois_chain_rule_t(std::vector<LoopRec> &run, size_t at) {
   ensure_partials((size_t)g.blocks() * 8);
   PoisChainPtrs<T> c;
   DatView pv = view_of(P);
-  c.pnew = Ptr<T>{(T *)spare_base(P, R), pv.sy, pv.sz};
+  c.pnew = Ptr<T>{(T *)spare_base(P, R, true), pv.sy, pv.sz};
   c.pold = ptr_of<const T>(P);
   c.r = ptr_of<const T>(Rr);
   c.w = ptr_of<T>(W);
@@ -346,7 +346,7 @@ void launch_jacobi_chain(const LoopRec &cp, const LoopRec &jac, const Range3 &R)
   ensure_partials((size_t)gx * gy * sizeof(T));
   JacPtrs<T> c;
   DatView v = view_of(An);
-  c.out = Ptr<T>{(T *)spare_base(An, R), v.sy, v.sz};
+  c.out = Ptr<T>{(T *)spare_base(An, R, true), v.sy, v.sz};
   c.A = ptr_of<T>(A);
   c.An = ptr_of<const T>(An);
   const RedCtl ctl = with_host_fold(jac.ctl, gx * gy, 1, sizeof(T) == 8 ? DT_F64 : DT_F32);

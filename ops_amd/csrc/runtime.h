@@ -338,12 +338,13 @@ void flush_for(ops_reduction h);
 void deps_from_args(LoopRec &rec, const ops_arg *args, int n);
 // Double buffering for fused chains that rewrite a dat its own stencil reads
 // over a range r: spare_base(d, r) is point (0,...,0) of a second allocation
-// of d that equals d's current buffer everywhere outside r (copied in full
-// when that is not known to hold); the fused kernel then writes all of r
-// into it and swap_spare(d, r) makes it d's buffer.  The old buffer, now the
+// of d that equals d's current buffer everywhere outside r (copied when that
+// is not known to hold: in full, or, for a kernel that writes_all of r
+// whatever its values, outside r only); the fused kernel then writes r into
+// it and swap_spare(d, r) makes it d's buffer.  The old buffer, now the
 // spare, differs from the new one only inside r, so a following chain over
 // the same r needs no copy.  Any other write to d marks the spare out of date.
-char *spare_base(ops_dat d, const Range3 &r);
+char *spare_base(ops_dat d, const Range3 &r, bool writes_all = false);
 void swap_spare(ops_dat d, const Range3 &r);
 void note_external_write(ops_dat d);
 void trid_noalloc_setup(int dev);  // trid.hip: per-device address of the no-allocation scratch

@@ -219,3 +219,41 @@ def test_poisson_columns_tile_edges(gpu_ops, n, dtype):
     ref = dtype(6) * p - (e[c, c, :-2] + e[c, c, 2:]) - (e[c, :-2, c] + e[c, 2:, c]) - (e[:-2, c, c] + e[2:, c, c])
     assert np.array_equal(w, ref)
     assert abs(out[0][0][-1] - np.sum(w.astype(np.float64) * p)) <= 1e-12 * np.sum(np.abs(w.astype(np.float64) * p))
+
+
+@pytest.mark.parametrize("n", [(37, 20, 11), (130, 17, 9)])
+def test_chain_buffers_keep_what_lies_outside_the_range(gpu_ops, n):
+    """p's two buffers after chains over the interior and over a part of it,
+    with its halo and interior rewritten in between: the whole array, halos
+    included, as the separate loops leave it"""
+    ops = gpu_ops
+    blk, s0, rg = _setup(ops, n)
+    nx, ny, nz = n
+    part = [2, nx - 3, 1, ny - 2, 3, nz - 1]
+    sp = ops.ops_decl_stencil(3, 7, O_pts(3), "sp")
+    R, RW, W = ops.OPS_READ, ops.OPS_RW, ops.OPS_WRITE
+    out = []
+    for level in (0, 2):
+        rng = np.random.RandomState(9)
+        ops.ops_mi_set_fusion(level)
+        D = {k: ops.ops_decl_dat(blk, list(n), dtype=np.float32, name=k) for k in "rpw"}
+        for d in D.values():
+            ops.set_ext(d, rng.rand(nz + 2, ny + 2, nx + 2).astype(np.float32))
+        red = ops.ops_decl_reduction_handle(8, "double", "pw")
+        A = lambda k, s, acc: ops.ops_arg_dat(D[k], 1, s, "float", acc)
+        got = []
+        for step, rng6 in enumerate([rg, rg, part, part, rg, part, rg]):
+            if step in (1, 3, 4):
+                ops.set_ext(D["p"], rng.rand(nz + 2, ny + 2, nx + 2).astype(np.float32))
+            ops.ops_par_loop("mp_p_kernel", "p", blk, 3, rng6, A("p", s0, RW), A("r", s0, R),
+                             ops.ops_arg_gbl(0.5, 1, "float"), ops.ops_arg_gbl(0.25, 1, "float"))
+            ops.ops_par_loop("poisson_calc_w_reduce_kernel", "w", blk, 3, rng6, A("w", s0, W), A("p", sp, R),
+                             ops.ops_arg_reduce(red, 1, "double", ops.OPS_INC))
+            ops.ops_reduction_result(red)
+            got += [ops.get_ext(D["p"]), ops.get_ext(D["w"])]
+        out.append(got)
+        for d in D.values():
+            ops.ops_free_dat(d)
+    ops.ops_mi_set_fusion(2)
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
