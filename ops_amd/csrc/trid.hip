@@ -184,7 +184,8 @@ __global__ __launch_bounds__(256) void k_thomas(const T *__restrict__ a, const T
 
 // Solves along x (element stride 1).  One thread per system would make each
 // load of a wave touch 64 rows (64 cache lines); here a one-wave workgroup
-// takes 64 systems and moves them through LDS in chunks of kChunk steps: the
+// takes NS systems (64, or 32 where 64 would leave SIMDs without a wave) and
+// moves them through LDS in chunks of kChunk steps: the
 // wave loads a chunk of a, b, c, d with row-contiguous V-wide loads (kChunk/V
 // lanes per system), stores it transposed ([step][system]) in LDS, and each
 // lane runs the same recurrence as k_thomas on its system from LDS, writing
@@ -194,21 +195,21 @@ __global__ __launch_bounds__(256) void k_thomas(const T *__restrict__ a, const T
 // row-contiguous stores.  Same operations in the same order as k_thomas.
 constexpr int kChunk = 16;
 
-template <class T, int V>
+template <class T, int V, int NS>
 struct XChunk {
   static constexpr int kLanesPerSys = kChunk / V;      // lanes covering one system's chunk
   static constexpr int kSysPerLoad = 64 / kLanesPerSys;  // systems per wave-wide load
-  static constexpr int kLoads = 64 / kSysPerLoad;        // loads per array per chunk
+  static constexpr int kLoads = NS / kSysPerLoad;        // loads per array per chunk
 };
 
-template <class T, int V, bool INC>
+template <class T, int V, int NS, bool INC>
 __global__ __launch_bounds__(64) void k_thomas_x(const T *__restrict__ a, const T *__restrict__ b,
                                                  const T *__restrict__ c, T *__restrict__ d, T *__restrict__ u,
                                                  T *__restrict__ cs, T *__restrict__ ds, LineGeo g) {
-  using XC = XChunk<T, V>;
-  __shared__ T LA[kChunk][65], LB[kChunk][65], LC[kChunk][65], LD[kChunk][65];
+  using XC = XChunk<T, V, NS>;
+  __shared__ T LA[kChunk][NS + 1], LB[kChunk][NS + 1], LC[kChunk][NS + 1], LD[kChunk][NS + 1];
   const int lane = (int)threadIdx.x;
-  const long first = (long)blockIdx.x * 64;
+  const long first = (long)blockIdx.x * NS;
   const long id = first + lane;  // this lane's system in the recurrence
   const long L = g.count, n = g.n;
   // the systems and chunk positions this lane covers in row-contiguous loads
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(64) void k_thomas_x(const T *__restrict__ a, const 
   }
   T ra[XC::kLoads][V], rb[XC::kLoads][V], rc[XC::kLoads][V], rd[XC::kLoads][V];
   // every system of the workgroup exists (workgroup-uniform)
-  const bool all_rows = first + 64 <= L;
+  const bool all_rows = first + NS <= L;
   auto load_chunk = [&](long i0) {
     if (all_rows && i0 + kChunk <= n) {
       // a full chunk: no per-row branches, so the loads of all rows are in
@@ -288,7 +289,7 @@ __global__ __launch_bounds__(64) void k_thomas_x(const T *__restrict__ a, const 
       }
     }
   };
-  const bool live = id < L;
+  const bool live = lane < NS && id < L;
   T cprev = 0, dprev = 0;
   load_chunk(0);
   for (long i0 = 0; i0 < n; i0 += kChunk) {
@@ -680,32 +681,45 @@ void trid_run(int ndim, int solvedim, int *range, ops_dat a, ops_dat b, ops_dat 
   } else {
     size_t sb = (size_t)g.n * g.count * es;
     char *scr = fixed_scr ? fixed_scr : (char *)trid_scratch(2 * sb);
-    int nblk = (int)((g.count + 255) / 256);
+    // one-wave workgroups while each then has a CU to itself (100^3 in FP64:
+    // 29 us instead of 46 in 40 workgroups of four waves); beyond that four
+    // waves share a CU better (45 000 systems of 203 in FP32: 83 and 91 us)
+    const int tpb = g.count <= 64L * inst().num_cus ? 64 : 256;
+    int nblk = (int)((g.count + tpb - 1) / tpb);
     if (solvedim == 0) {
       // x solves: LDS-staged chunks, 16-byte row loads when every array's
-      // rows start 16-byte aligned
-      bool v16 = g.s0 % 2 == 0 && g.s1 % 2 == 0;
+      // rows start 16-byte aligned (30 450 systems of 301 in FP32: 143 us
+      // instead of 164 with single elements)
+      const long per16 = 16 / (long)es;
+      bool v16 = g.s0 % per16 == 0 && g.s1 % per16 == 0;
       for (char *p : {pa, pb, pc, pd, pu})
         if (p && (uintptr_t)p % 16 != 0) v16 = false;
-      if (dt == DT_F32) v16 = false;
-      const int nw = (int)((g.count + 63) / 64);
+      // half-filled waves (32 systems) while each of those finds a SIMD of its
+      // own: 30 450 systems of 301 in FP64 take 147 us instead of 201, in FP32
+      // 123 instead of 143, 10 000 of 100 40 instead of 43.  Past that the
+      // fuller waves win: 40 000 systems of 301 in FP64 180 us against 238,
+      // 65 536 of 256 217 against 261
+      const bool half = g.count <= 128L * inst().num_cus;
+      const int nw = (int)((g.count + (half ? 31 : 63)) / (half ? 32 : 64));
       launch([&](hipStream_t s) {
-        if (dt == DT_F64) {
-          double *A = (double *)pa, *B = (double *)pb, *C = (double *)pc, *D = (double *)pd, *U = (double *)pu;
-          double *CS = (double *)scr, *DS = (double *)(scr + sb);
-          if (v16) {
-            if (u) hipLaunchKernelGGL((k_thomas_x<double, 2, true>), dim3(nw), dim3(64), 0, s, A, B, C, D, U, CS, DS, g);
-            else hipLaunchKernelGGL((k_thomas_x<double, 2, false>), dim3(nw), dim3(64), 0, s, A, B, C, D, U, CS, DS, g);
-          } else {
-            if (u) hipLaunchKernelGGL((k_thomas_x<double, 1, true>), dim3(nw), dim3(64), 0, s, A, B, C, D, U, CS, DS, g);
-            else hipLaunchKernelGGL((k_thomas_x<double, 1, false>), dim3(nw), dim3(64), 0, s, A, B, C, D, U, CS, DS, g);
-          }
-        } else {
-          float *A = (float *)pa, *B = (float *)pb, *C = (float *)pc, *D = (float *)pd, *U = (float *)pu;
-          float *CS = (float *)scr, *DS = (float *)(scr + sb);
-          if (u) hipLaunchKernelGGL((k_thomas_x<float, 1, true>), dim3(nw), dim3(64), 0, s, A, B, C, D, U, CS, DS, g);
-          else hipLaunchKernelGGL((k_thomas_x<float, 1, false>), dim3(nw), dim3(64), 0, s, A, B, C, D, U, CS, DS, g);
-        }
+        auto go = [&](auto v, auto ns, auto *t) {
+          using T = std::remove_pointer_t<decltype(t)>;
+          constexpr int V = decltype(v)::value, NS = decltype(ns)::value;
+          hipLaunchKernelGGL((u ? k_thomas_x<T, V, NS, true> : k_thomas_x<T, V, NS, false>), dim3(nw), dim3(64), 0, s,
+                             (const T *)pa, (const T *)pb, (const T *)pc, (T *)pd, (T *)pu, (T *)scr,
+                             (T *)(scr + sb), g);
+        };
+        auto width = [&](auto ns, auto *t) {
+          using T = std::remove_pointer_t<decltype(t)>;
+          if (v16) go(std::integral_constant<int, 16 / (int)sizeof(T)>{}, ns, t);
+          else go(std::integral_constant<int, 1>{}, ns, t);
+        };
+        auto type = [&](auto ns) {
+          if (dt == DT_F64) width(ns, (double *)nullptr);
+          else width(ns, (float *)nullptr);
+        };
+        if (half) type(std::integral_constant<int, 32>{});
+        else type(std::integral_constant<int, 64>{});
       });
       mark_device_dirty(u ? u : d);
       note_external_write(u ? u : d);
@@ -713,11 +727,11 @@ void trid_run(int ndim, int solvedim, int *range, ops_dat a, ops_dat b, ops_dat 
     }
     launch([&](hipStream_t s) {
       if (dt == DT_F64) {
-        if (u) hipLaunchKernelGGL((k_thomas<double, true, kPre>), dim3(nblk), dim3(256), 0, s, (double *)pa, (double *)pb, (double *)pc, (double *)pd, (double *)pu, (double *)scr, (double *)(scr + sb), g);
-        else hipLaunchKernelGGL((k_thomas<double, false, kPre>), dim3(nblk), dim3(256), 0, s, (double *)pa, (double *)pb, (double *)pc, (double *)pd, (double *)pu, (double *)scr, (double *)(scr + sb), g);
+        if (u) hipLaunchKernelGGL((k_thomas<double, true, kPre>), dim3(nblk), dim3(tpb), 0, s, (double *)pa, (double *)pb, (double *)pc, (double *)pd, (double *)pu, (double *)scr, (double *)(scr + sb), g);
+        else hipLaunchKernelGGL((k_thomas<double, false, kPre>), dim3(nblk), dim3(tpb), 0, s, (double *)pa, (double *)pb, (double *)pc, (double *)pd, (double *)pu, (double *)scr, (double *)(scr + sb), g);
       } else {
-        if (u) hipLaunchKernelGGL((k_thomas<float, true, kPre>), dim3(nblk), dim3(256), 0, s, (float *)pa, (float *)pb, (float *)pc, (float *)pd, (float *)pu, (float *)scr, (float *)(scr + sb), g);
-        else hipLaunchKernelGGL((k_thomas<float, false, kPre>), dim3(nblk), dim3(256), 0, s, (float *)pa, (float *)pb, (float *)pc, (float *)pd, (float *)pu, (float *)scr, (float *)(scr + sb), g);
+        if (u) hipLaunchKernelGGL((k_thomas<float, true, kPre>), dim3(nblk), dim3(tpb), 0, s, (float *)pa, (float *)pb, (float *)pc, (float *)pd, (float *)pu, (float *)scr, (float *)(scr + sb), g);
+        else hipLaunchKernelGGL((k_thomas<float, false, kPre>), dim3(nblk), dim3(tpb), 0, s, (float *)pa, (float *)pb, (float *)pc, (float *)pd, (float *)pu, (float *)scr, (float *)(scr + sb), g);
       }
     });
   }

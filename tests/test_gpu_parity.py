@@ -692,6 +692,39 @@ def test_stencil27_column_bit_exact(gpu_ops, n):
     ops.ops_free_dat(o)
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n,lo,hi", [
+    ((17, 256, 128), 0, 0), ((20, 257, 128), 0, 0), ((128, 5, 128), 0, 0), ((129, 4, 128), 0, 0),
+    ((48, 33, 3), 0, 0), ((35, 31, 2), 0, 0), ((40, 13, 5), 4, 1), ((40, 13, 5), 1, 2), ((1, 7, 3), 0, 0)])
+def test_thomas_workgroup_shapes_bit_exact(gpu_ops, dtype, n, lo, hi):
+    """system counts on both sides of the switches between workgroup shapes
+    (128 systems per CU along x, 64 along y and z, at 256 CUs) and of whole
+    waves; lengths around a chunk of 16; ranges that start on and off 16 bytes"""
+    ops = gpu_ops
+    rng = np.random.RandomState(6)
+    shape = n[::-1]
+    blk = ops.ops_decl_block(3, "thomasshape")
+    D = {k: ops.ops_decl_dat(blk, list(n), dtype=dtype, name=k) for k in "abcdu"}
+    ctx = ops.TridParams(blk)
+    rg = [lo, n[0] - hi, 0, n[1], 0, n[2]]
+    dims = [n[0] - hi - lo, n[1], n[2]]
+    a, c = rng.rand(*shape).astype(dtype) - 1, rng.rand(*shape).astype(dtype) - 1
+    b = (abs(a) + abs(c) + dtype(0.1) + rng.rand(*shape).astype(dtype)).astype(dtype)
+    d, u = rng.rand(*shape).astype(dtype), rng.rand(*shape).astype(dtype)
+    for k, v in zip("abcdu", (a, b, c, d, u)):
+        ops.ops_dat_set_data(D[k], v)
+    flat = lambda v: v.reshape(-1)[lo:]
+    for sd in range(3):
+        O.thomas_batch(3, sd, dims, list(n), flat(a), flat(b), flat(c), flat(d).copy(), flat(u), nthreads=NT)
+        ops.ops_tridMultiDimBatch_Inc(3, sd, rg, D["a"], D["b"], D["c"], D["d"], D["u"], ctx)
+        assert np.array_equal(ops.ops_dat_fetch_data(D["u"]), u), sd
+        O.thomas_batch(3, sd, dims, list(n), flat(a), flat(b), flat(c), flat(d), None, nthreads=NT)
+        ops.ops_tridMultiDimBatch(3, sd, rg, D["a"], D["b"], D["c"], D["d"], ctx)
+        assert np.array_equal(ops.ops_dat_fetch_data(D["d"]), d), sd
+    for q in D.values():
+        ops.ops_free_dat(q)
+
+
 def _pcr_numpy(a, b, c, d):
     """parallel cyclic reduction along the last axis in the arrays' own type,
     with the operations and order of the kernel and the oracle"""
