@@ -22,6 +22,7 @@
 // separate loops.
 #include "column.h"
 #include "engine.h"
+#include "heat2.h"
 
 using namespace opsmi;
 
@@ -145,13 +146,72 @@ int axpy_axpby_rule(std::vector<LoopRec> &run, size_t at, hipStream_t s) {
   return 2;
 }
 
+// The chain in 2D, on k_heat2 (same partial sums as calc_w alone): 64 bytes a
+// point instead of 40 (the pair) + 32 (calc_w).
+int cg_chain2_rule(std::vector<LoopRec> &run, size_t at, hipStream_t) {
+  size_t i = at;
+  const LoopRec *ax = nullptr;
+  if (i < run.size() && run[i].kind == LK_AXPY) ax = &run[i++];
+  if (i + 1 >= run.size()) return 0;
+  const LoopRec &bp = run[i], &cw = run[i + 1];
+  if (bp.kind != LK_AXPBY || cw.kind != LK_HEAT_W2 || cw.dims != 2 || bp.dims != 2) return 0;
+  const ops_dat P = bp.d[0], Rr = bp.d[1], W = cw.d[0], Kx = cw.d[1], Ky = cw.d[2];
+  if (cw.d[4] != P || P == Rr || W == P || W == Rr) return 0;
+  if (Kx == P || Ky == P || Kx == W || Ky == W) return 0;
+  const Range3 R = cw.range;
+  if (!same_range(bp.range, R) || R.npts() <= 0 || cw.ctl.slot == nullptr) return 0;
+  if (!heat2_ok(R, {P, Rr, W, Kx, Ky})) return 0;
+  ops_dat U = nullptr;
+  if (ax) {
+    // an axpy that this pass cannot take with it leaves the three to the other rules
+    U = ax->d[0];
+    if (ax->d[1] != P || ax->dims != 2 || !same_range(ax->range, R) || !heat2_ok(R, {U})) return 0;
+    for (ops_dat d : {P, Rr, W, Kx, Ky})
+      if (U == d) return 0;
+  }
+  if (!have_spare(P)) return 0;
+  Heat2Args f{};
+  const DatView pv = view_of(P);
+  f.pnew = Ptr<double>{(double *)spare_base(P, R, true), pv.sy, pv.sz};
+  f.p = ptr_of<const double>(P);
+  f.rr = ptr_of<const double>(Rr);
+  f.w = ptr_of<double>(W);
+  f.Kx = ptr_of<const double>(Kx);
+  f.Ky = ptr_of<const double>(Ky);
+  if (U) f.u = ptr_of<double>(U);
+  f.alpha_u = ax ? ax->g[0] : 0.0;
+  f.a = bp.g[0];
+  f.b = bp.g[1];
+  f.rx = cw.g[0];
+  f.ry = cw.g[1];
+  const unsigned parts = heat2_parts(R);
+  ensure_partials((size_t)parts * 8);
+  const RedCtl ctl = with_host_fold(cw.ctl, parts, 1, DT_F64);
+  const double bytes = (ax ? ax->bytes : 0.0) + bp.bytes + cw.bytes;
+  const bool nt = 7.0 * 8.0 * R.npts() >= kNtLoadBytes;
+  auto kern = !ax ? k_heat2<HEAT2_CHAIN> : nt ? k_heat2<HEAT2_CHAIN_AXPY, true> : k_heat2<HEAT2_CHAIN_AXPY>;
+  run_loop(ax ? "cg_chain(axpy+axpby+calc_w)" : "cg_chain(axpby+calc_w)", bytes, [&](hipStream_t st) {
+    hipLaunchKernelGGL(kern, heat2_grid(R), dim3(kWave, kWavesPerBlock), 0, st, f, R, heat2_tiles(R), ctl);
+    launch_red_finish<double, OPS_INC, 1>(ctl, parts, st);
+  });
+  swap_spare(P, R);
+  if (U) note_external_write(U);
+  note_external_write(W);
+  if (ax) note_fused(ax->name.c_str(), ax->bytes);
+  note_fused(bp.name.c_str(), bp.bytes);
+  note_fused(cw.name.c_str(), cw.bytes);
+  return (int)(i + 2 - at);
+}
+
 // The three-loop chain moves 72 instead of 80 bytes per point: at 512^3 it
 // measured 1853 us against 1025 + 934 us for calc_w and the pair (2093 us
 // when it formed p_new as each load arrived, which made every load wait).
 // It runs at fusion level 2 (the default); at level 1 the pair rule takes the
 // axpy + axpby and calc_w runs alone.
 int cg_chain_rule_level2(std::vector<LoopRec> &run, size_t at, hipStream_t s) {
-  return inst().fusion >= 2 ? cg_chain_rule(run, at, s) : 0;
+  if (inst().fusion < 2) return 0;
+  if (const int taken = cg_chain_rule(run, at, s)) return taken;
+  return cg_chain2_rule(run, at, s);
 }
 
 // Constant-coefficient Poisson chains (poisson3_chain_column_v), on the

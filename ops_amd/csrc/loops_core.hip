@@ -6,6 +6,7 @@
 // for bit; sums differ only by reduction order.
 #include "column.h"
 #include "engine.h"
+#include "heat2.h"
 #include "heat_tile.h"
 
 using namespace opsmi;
@@ -276,6 +277,36 @@ LoopRec make_heat3_loop(const char *name, const ops_arg *args, int nargs, const 
                        ptr_of<const double>(Kx.dat), ptr_of<const double>(Ky.dat), ptr_of<const double>(Kz.dat),
                        ptr_of<const double>(p.dat), rx, ry, rz, r, g.chunk, c);
     if (!INIT) launch_red_finish<double, OPS_INC, 1>(c, g.blocks(), s);
+  };
+  return rec;
+}
+
+// Queue record of the 2D operator on k_heat2 (heat2_ok holds)
+template <bool INIT>
+LoopRec make_heat2_loop(const char *name, const ops_arg *args, int nargs, const Range3 &r, ops_arg w, ops_arg rr,
+                        ops_arg Kx, ops_arg Ky, ops_arg p, double rx, double ry, const ops_arg *red) {
+  LoopRec rec;
+  rec.name = name;
+  rec.range = r;
+  rec.bytes = transfer_bytes(args, nargs, r);
+  deps_from_args(rec, args, nargs);
+  const unsigned parts = heat2_parts(r);
+  RedCtl ctl{};
+  if (!INIT) ctl = red_prepare(*red, 1, DT_F64, parts);
+  rec.ctl = ctl;
+  rec.launch = [=](hipStream_t s) {
+    const RedCtl c = INIT ? with_scratch(ctl) : with_host_fold(ctl, parts, 1, DT_F64);
+    Heat2Args f{};
+    f.w = ptr_of<double>(w.dat);
+    if (INIT) f.r = ptr_of<double>(rr.dat);
+    f.Kx = ptr_of<const double>(Kx.dat);
+    f.Ky = ptr_of<const double>(Ky.dat);
+    f.p = ptr_of<const double>(p.dat);
+    f.rx = rx;
+    f.ry = ry;
+    hipLaunchKernelGGL((k_heat2<(INIT ? HEAT2_INIT : HEAT2_W)>), heat2_grid(r), dim3(kWave, kWavesPerBlock), 0, s, f,
+                       r, heat2_tiles(r), c);
+    if (!INIT) launch_red_finish<double, OPS_INC, 1>(c, parts, s);
   };
   return rec;
 }
@@ -774,7 +805,10 @@ void ops_par_loop_tea_leaf_common_init_kernel(const char *name, ops_block block,
                         nullptr);
   need_dim(name, dim, 2);
   const double vx = gbl<double>(rx), vy = gbl<double>(ry);
-  LAUNCH(r, CommonInit<2>{PD(w), PD(rr), PCD(Kx), PCD(Ky), Ptr<const double>{nullptr, 0, 0}, PCD(u), vx, vy, 0.0});
+  if (r.npts() > 0 && heat2_ok(r, {w.dat, rr.dat, Kx.dat, Ky.dat, u.dat}))
+    enqueue(make_heat2_loop<true>(name, args, nargs, r, w, rr, Kx, Ky, u, vx, vy, nullptr));
+  else
+    LAUNCH(r, CommonInit<2>{PD(w), PD(rr), PCD(Kx), PCD(Ky), Ptr<const double>{nullptr, 0, 0}, PCD(u), vx, vy, 0.0});
   finish_loop(args, nargs);
   OPSMI_API_END()
 }
@@ -807,7 +841,22 @@ void ops_par_loop_tea_leaf_cg_calc_w_reduce_kernel(const char *name, ops_block b
                         nullptr);
   need_dim(name, dim, 2);
   const double vx = gbl<double>(rx), vy = gbl<double>(ry);
-  LAUNCH_RED(r, pw, CalcW<2>{PD(w), PCD(Kx), PCD(Ky), Ptr<const double>{nullptr, 0, 0}, PCD(p), vx, vy, 0.0});
+  const bool vec = r.npts() > 0 && heat2_ok(r, {w.dat, Kx.dat, Ky.dat, p.dat});
+  const Ptr<const double> none{nullptr, 0, 0};
+  LoopRec rec = vec ? make_heat2_loop<false>(name, args, nargs, r, w, w, Kx, Ky, p, vx, vy, &pw)
+                    : make_loop(name, args, nargs, r,
+                                [=] { return CalcW<2>{PD(w), PCD(Kx), PCD(Ky), none, PCD(p), vx, vy, 0.0}; }, &pw);
+  if (vec) {
+    rec.kind = LK_HEAT_W2;
+    rec.dims = dim;
+    rec.d[0] = w.dat;
+    rec.d[1] = Kx.dat;
+    rec.d[2] = Ky.dat;
+    rec.d[4] = p.dat;
+    rec.g[0] = vx;
+    rec.g[1] = vy;
+  }
+  enqueue(std::move(rec));
   finish_loop(args, nargs);
   OPSMI_API_END()
 }

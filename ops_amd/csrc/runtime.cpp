@@ -695,14 +695,26 @@ static void set_spare_range(DatImpl *m, const Range3 &r) {
   memcpy(m->spare_range, rr, sizeof(rr));
 }
 
+bool have_spare(ops_dat d) {
+  DatImpl *m = (DatImpl *)d->impl;
+  if (m->spare) return true;
+  const size_t lead = (size_t)(d->data_d - m->alloc);
+  const hipError_t e = hipMalloc(&m->spare, d->mem + lead + 256);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    m->spare = nullptr;
+    return false;
+  }
+  OPSMI_HIP(e);
+  m->spare_synced = false;
+  return true;
+}
+
 char *spare_base(ops_dat d, const Range3 &r, bool writes_all) {
   Instance &I = inst();
   DatImpl *m = (DatImpl *)d->impl;
   size_t lead = (size_t)(d->data_d - m->alloc);
-  if (!m->spare) {
-    OPSMI_HIP(hipMalloc(&m->spare, d->mem + lead + 256));
-    m->spare_synced = false;
-  }
+  if (!have_spare(d)) OPSMI_HIP(hipErrorOutOfMemory);
   // the spare may differ from the buffer inside the last swapped range only.
   // A pass that writes all of r into the spare needs no more of it brought up
   // to date than what lies outside, a halo's worth (512^3: 778 us for the

@@ -305,6 +305,7 @@ enum LoopKind {
   LK_AXPY,       // tea_leaf_axpy_kernel: u = u + a p
   LK_AXPBY,      // tea_leaf_axpby_kernel: u = a u + b p
   LK_HEAT_W3,    // tea_leaf_cg_calc_w_reduce_kernel (3D): w = A p, pw
+  LK_HEAT_W2,    // tea_leaf_cg_calc_w_reduce_kernel (2D, k_heat2 form): w = A p, pw
   LK_POISSON_W3, // poisson_calc_w_reduce_kernel (3D column form): w = A p, pw; g[0] = element bytes
   LK_MP_E,       // mp_e_update_kernel: e = e + a p (float)
   LK_MP_P,       // mp_p_kernel: p = mi rr + b p (float)
@@ -346,6 +347,8 @@ void deps_from_args(LoopRec &rec, const ops_arg *args, int n);
 // the same r needs no copy.  Any other write to d marks the spare out of date.
 char *spare_base(ops_dat d, const Range3 &r, bool writes_all = false);
 void swap_spare(ops_dat d, const Range3 &r);
+// allocates d's spare if it has none; false when there is no memory for it
+bool have_spare(ops_dat d);
 void note_external_write(ops_dat d);
 void trid_noalloc_setup(int dev);  // trid.hip: per-device address of the no-allocation scratch
 // counts a loop that ran inside a fused kernel (its time is the fused entry's)
