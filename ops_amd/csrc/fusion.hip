@@ -63,16 +63,17 @@ int cg_chain_rule(std::vector<LoopRec> &run, size_t at, hipStream_t s) {
   ops_dat U = nullptr;
   if (ax) {
     U = ax->d[0];
-    // the deferred axpy must read this p_old and touch nothing else in the chain
+    // the deferred axpy must read this p_old and touch nothing else in the
+    // chain; any other runs alone first
     if (ax->d[1] != P || !same_range(ax->range, cw.range) || U == P || U == Rr || U == W || U == Kx ||
         U == Ky || U == Kz || ax->dims != 3)
-      ax = nullptr, U = nullptr;
+      return 0;
   }
   const Range3 R = cw.range;
   // the column kernel takes 16-byte loads from every array
   for (ops_dat d : {P, Rr, W, Kx, Ky, Kz})
     if (!vec16_ok(d, R.x0)) return 0;
-  if (U && !vec16_ok(U, R.x0)) ax = nullptr, U = nullptr;
+  if (U && !vec16_ok(U, R.x0)) return 0;
   if (!use_vec() || cw.ctl.slot == nullptr) return 0;
   constexpr int V = 2;
   const ColGrid g = heat_column_grid(R, V * kWave, kHeatRows);
@@ -163,7 +164,7 @@ int cg_chain2_rule(std::vector<LoopRec> &run, size_t at, hipStream_t) {
   if (!heat2_ok(R, {P, Rr, W, Kx, Ky})) return 0;
   ops_dat U = nullptr;
   if (ax) {
-    // an axpy that this pass cannot take with it leaves the three to the other rules
+    // as in 3D: an axpy that cannot join runs alone first
     U = ax->d[0];
     if (ax->d[1] != P || ax->dims != 2 || !same_range(ax->range, R) || !heat2_ok(R, {U})) return 0;
     for (ops_dat d : {P, Rr, W, Kx, Ky})
@@ -251,12 +252,12 @@ int pois_chain_rule_t(std::vector<LoopRec> &run, size_t at) {
   if (ax) {
     U = ax->d[0];
     if (ax->d[1] != P || !same_range(ax->range, cw.range) || U == P || U == Rr || U == W || ax->dims != 3)
-      ax = nullptr, U = nullptr;
+      return 0;
   }
   const Range3 R = cw.range;
   for (ops_dat d : {P, Rr, W})
     if (!vec16_ok(d, R.x0)) return 0;
-  if (U && !vec16_ok(U, R.x0)) ax = nullptr, U = nullptr;
+  if (U && !vec16_ok(U, R.x0)) return 0;
   if (!use_vec() || cw.ctl.slot == nullptr) return 0;
   constexpr int V = 16 / (int)sizeof(T);
   const ColGrid g = column_grid(R, V * kWave, kHeatRows);

@@ -106,6 +106,41 @@ def test_fused_cg_chain_bit_identical(gpu_ops, n):
         assert np.array_equal(u0, u)
 
 
+@pytest.mark.parametrize("op", ["heat2", "heat3", "poisson3"])
+def test_axpy_that_does_not_join_the_chain_still_runs(gpu_ops, op):
+    """r -= 0.5 w as an axpy right before the axpby and the operator: it is not
+    the chain's u update, and must not be lost"""
+    from opshelp import heat_setup_py
+    ops = gpu_ops
+    nd = 2 if op == "heat2" else 3
+    n = (130, 20, 1) if nd == 2 else (130, 12, 9)
+    K, rhs = O.heat_inputs(24, nd, *n)
+    R, W, RW, INC = ops.OPS_READ, ops.OPS_WRITE, ops.OPS_RW, ops.OPS_INC
+    out = []
+    for level in (0, 2):
+        ops.ops_mi_set_fusion(level)
+        blk, D, st, red, inner, _ = heat_setup_py(ops, nd, n, K, rhs)
+        A = lambda q, s, acc: ops.ops_arg_dat(D[q], 1, st[s], "double", acc)
+        g = lambda v: ops.ops_arg_gbl(v, 1, "double")
+        coef = [A("K" + c, "s" + c, R) for c in "xyz"[:nd]]
+        sums = []
+        for it in range(3):
+            ops.ops_par_loop("tea_leaf_axpy_kernel", "axpy", blk, nd, inner, A("r", "s0", INC), A("w", "s0", R), g(-0.5))
+            ops.ops_par_loop("tea_leaf_axpby_kernel", "axpby", blk, nd, inner, A("p", "s0", RW), A("r", "s0", R),
+                             g(0.25), g(1.0))
+            rd = ops.ops_arg_reduce(red, 1, "double", INC)
+            if op == "poisson3":
+                ops.ops_par_loop("poisson_calc_w_reduce_kernel", "w", blk, nd, inner, A("w", "s0", W), A("p", "sp", R), rd)
+            else:
+                ops.ops_par_loop("tea_leaf_cg_calc_w_reduce_kernel" + ("" if nd == 2 else "_3d"), "w", blk, nd, inner,
+                                 A("w", "s0", W), *coef, A("p", "sp", R), *[g(1.0)] * nd, rd)
+            sums.append(ops.ops_reduction_result(red))
+        out.append([np.array(sums)] + [ops.ops_dat_fetch_data(D[k]) for k in "rpw"])
+    ops.ops_mi_set_fusion(2)
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("n", [(48, 40, 33), (130, 66, 40), (260, 37, 21)])
 def test_fused_poisson_chains_bit_identical(gpu_ops, n):
     """The constant-coefficient chains: FP64 CG (axpy + axpby + Poisson
