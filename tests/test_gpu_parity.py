@@ -725,6 +725,26 @@ def test_thomas_workgroup_shapes_bit_exact(gpu_ops, dtype, n, lo, hi):
         ops.ops_free_dat(q)
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n,lo,hi", [((257, 9), 0, 0), ((257, 9), 1, 0), ((255, 5), 4, 3), ((3, 2), 0, 0),
+                                     ((700, 70, 3), 4, 1), ((2, 3, 4), 1, 0), ((700, 440, 230), 0, 1)])
+def test_set_zero_ranges(gpu_ops, dtype, n, lo, hi):
+    """ranges that start on and off 16 bytes and end inside a lane; the last
+    one, in FP64, is larger than the caches: zeros inside, the rest untouched"""
+    ops = gpu_ops
+    nd = len(n)
+    blk = ops.ops_decl_block(nd, "zero")
+    s0 = ops.ops_decl_stencil(nd, 1, [0] * nd, "0")
+    a = ops.ops_decl_dat(blk, list(n), dtype=dtype, name="a")
+    v = np.full(n[::-1], 1.5, dtype)
+    ops.ops_dat_set_data(a, v)
+    ops.ops_par_loop("set_zero", "zero", blk, nd, [lo, n[0] - hi] + [q for m in n[1:] for q in (0, m)],
+                     ops.ops_arg_dat(a, 1, s0, "double" if dtype is np.float64 else "float", ops.OPS_WRITE))
+    v[..., lo:n[0] - hi] = 0
+    assert np.array_equal(ops.ops_dat_fetch_data(a), v)
+    ops.ops_free_dat(a)
+
+
 def _pcr_numpy(a, b, c, d):
     """parallel cyclic reduction along the last axis in the arrays' own type,
     with the operations and order of the kernel and the oracle"""
