@@ -5,9 +5,9 @@
  * ops_decl_block per problem, ops/c/src/core/ops_lib_core.cpp:376-434) are
  * solved together with unpreconditioned CG (the loop body of
  * apps/c/TeaLeaf/tea_leaf_cg.cpp:129-214: calc_w + p.w, u += alpha p and
- * r -= alpha w + r.r, p = beta p + r).  Every loop of the iteration is one
- * persistent launch over the tiles of all active blocks; the CG scalars stay
- * on the device, so iterations run without host round trips and are captured
+ * r -= alpha w + r.r, p = beta p + r).  An iteration is two persistent
+ * launches over the tiles of all active blocks; the CG scalars stay on the
+ * device, so iterations run without host round trips and are captured
  * in a HIP graph.  A continuous-batching scheduler admits queued solves
  * whenever a slot and HBM budget are free, between graph launches, while
  * the others keep iterating.  No counterpart in the reference library (its

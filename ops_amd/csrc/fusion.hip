@@ -7,7 +7,8 @@
 //     [tea_leaf_axpy_kernel        u = u + alpha p          (deferred from the
 //                                                            previous iteration)]
 //      tea_leaf_axpby_kernel       p = a p + b r
-//      tea_leaf_cg_calc_w_reduce   w = A p ; pw += w p      (3D, 7-point)
+//      tea_leaf_cg_calc_w_reduce   w = A p ; pw += w p      (3D, 7-point;
+//                                                            2D: cg_chain2_rule)
 // The lazy queue defers the axpy past the r.r result (nothing it depends on
 // changes) until the axpby that overwrites p needs it gone, so the three
 // loops meet here.  One z-marching column kernel (heat3_chain_column_v)
