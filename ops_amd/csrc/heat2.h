@@ -9,9 +9,10 @@
 // load per row.  Bound by memory: at 3001 x 2003 calc_w's 192 MB take 31 us
 // (6.2 TB/s, part of it from the Infinity Cache), common_init's 240 MB 47 us;
 // one point per lane and one row after the other (the general engine) took 46.5
-// and 52.6 us.  The chain's 385 MB take 73 us there and 2.3 GB 457 us at
-// 6000 x 6000 (pair and calc_w alone: 75 and 489 us); it needs 141 registers,
-// and squeezed into 128, for a fourth wave per SIMD, it spills and takes 494 us.
+// and 52.6 us.  The chain's 385 MB take 67.5 us there (73 without NT) and its
+// 2.3 GB 457 us at 6000 x 6000 (pair and calc_w alone: 72 and 489 us); it needs
+// 141 registers, and squeezed into 128, for a fourth wave per SIMD, it spills
+// and takes 494 us there.
 //
 // NT: Kx, Ky and u, which no other loop of the iteration touches, pass the
 // caches by, which leaves them to p, r and w: for a chain whose seven arrays
