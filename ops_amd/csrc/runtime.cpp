@@ -986,7 +986,13 @@ ops_dat ops_decl_dat_char(ops_block block, int dim, int *dsize, int *base, int *
   size_t lead = (A - ((size_t)(-d->d_m[0]) * unit) % A) % A;
   OPSMI_HIP(hipMalloc(&m->alloc, bytes + lead + A));
   d->data_d = m->alloc + lead;
-  OPSMI_HIP(hipMemset(m->alloc, 0, bytes + lead + A));
+  // cleared on the library's stream, which does not wait for the default one:
+  // an upload, and every later loop, comes after it.  What another stream may
+  // do with the new array (a caller's device buffer copied in below, kernels
+  // on a raw pointer) is preceded by a wait.
+  OPSMI_HIP(hipMemsetAsync(m->alloc, 0, bytes + lead + A, I.stream));
+  const bool on_device = data && device_pointer(data);
+  if (!data || on_device) OPSMI_HIP(hipStreamSynchronize(I.stream));
   if (data) {
     // user array: same layout without the x padding (SoA: one such array
     // per component, one after the other)
@@ -994,7 +1000,6 @@ ops_dat ops_decl_dat_char(ops_block block, int dim, int *dsize, int *base, int *
     size_t rows = 1;
     for (int n = 1; n < nd; n++) rows *= d->size[n];
     const int ncomp = m->soa ? dim : 1;
-    const bool on_device = device_pointer(data);
     for (int c = 0; c < ncomp; c++) {
       Box b;
       b.pitch = (long)(row + (size_t)d->x_pad * unit);

@@ -64,3 +64,20 @@ def test_declaration_with_data(gpu_ops, size):
     d = ops.ops_decl_dat(ops.ops_decl_block(nd, "withdata"), size, data=data, name="d")
     assert np.array_equal(ops.get_whole(d), data)
     ops.ops_free_dat(d)
+
+
+def test_declared_data_is_not_cleared_afterwards(gpu_ops):
+    """Clearing a new array is ordered before the upload into it, also while
+    the GPU is still clearing a large array declared just before (6 GiB, about
+    a millisecond).  The shell of zeros past the uploaded rows stays."""
+    ops = gpu_ops
+    blk = ops.ops_decl_block(2, "clearing")
+    data = np.arange(302 * 202, dtype=np.float64).reshape(202, 302) + 1
+    for _ in range(3):
+        big = ops.ops_decl_dat(blk, [16384, 49152], name="big")
+        d = ops.ops_decl_dat(blk, [300, 200], data=data, name="d")
+        assert np.array_equal(ops.get_whole(d), data)
+        corner = ops.ops_dat_fetch_data_slab(big, [16000, 16384, 49151, 49152])
+        assert not corner.any()
+        ops.ops_free_dat(d)
+        ops.ops_free_dat(big)
