@@ -1007,7 +1007,7 @@ ops_dat ops_decl_dat_char(ops_block block, int dim, int *dsize, int *base, int *
       b.base = d->data_d + (size_t)c * b.pitch * rows;
       b.width = upitch;
       b.rows = (unsigned)d->size[1];
-      b.planes = (unsigned)(rows / d->size[1]);
+      b.planes = (unsigned)(rows ? rows / d->size[1] : 0);  // a dimension may hold no points
       char *from = data + (size_t)c * upitch * rows;
       if (on_device) OPSMI_HIP(hipMemcpy2D(b.base, b.pitch, from, upitch, upitch, rows, hipMemcpyDefault));
       else box_copy(I.staging, I.stream, b, from, true);

@@ -81,3 +81,14 @@ def test_declared_data_is_not_cleared_afterwards(gpu_ops):
         assert not corner.any()
         ops.ops_free_dat(d)
         ops.ops_free_dat(big)
+
+
+@pytest.mark.parametrize("size", [[0], [5, 0], [0, 5], [4, 0, 3], [4, 3, 0]])
+def test_declaration_with_data_and_no_points(gpu_ops, size):
+    """an empty array (a dimension of no points and no halo) with a data
+    pointer: nothing to upload"""
+    ops = gpu_ops
+    nd = len(size)
+    blk = ops.ops_decl_block(nd, "empty")
+    d = ops.ops_decl_dat(blk, size, [0] * nd, [0] * nd, data=np.zeros(size[::-1]), name="d")
+    ops.ops_free_dat(d)
