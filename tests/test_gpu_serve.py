@@ -294,3 +294,44 @@ def test_mixed_at_tile_edges_equals_fp64(serve, kind, n):
     srv.close()
     assert out[a][0]["status"] == 1 and out[b][0]["status"] == 1
     assert np.max(np.abs(out[a][1] - out[b][1])) <= 1e-8 * np.max(np.abs(out[a][1]))
+
+
+def test_workgroups_with_tiles_of_several_solves(serve):
+    # about 9400 tiles on the grid's 2048 workgroups: each works on tiles of
+    # several solves, some on several of one.  The same bits as alone.
+    S = serve
+    reqs = [(0, 2300, False), (1, 130, False), (0, 2600, True), (1, 150, True), (0, 1700, False), (0, 2300, True)]
+    srv = S.Server(budget_bytes=2 << 30, max_slots=8)
+    ids = [srv.submit(k, n, seed=60 + q, max_iters=12, mixed=m) for q, (k, n, m) in enumerate(reqs)]
+    out = srv.run()
+    for q, (i, (k, n, m)) in enumerate(zip(ids, reqs)):
+        j = srv.submit(k, n, seed=60 + q, max_iters=12, mixed=m)
+        alone = srv.run()[j]
+        assert alone[0]["iters"] == out[i][0]["iters"] and alone[0]["rr"] == out[i][0]["rr"]
+        assert np.array_equal(alone[1], out[i][1]), (k, n, m)
+    srv.close()
+
+
+def test_iteration_time_grows_with_the_points(serve):
+    # 16384^2 has four times the points and tiles of 8192^2, both beyond the
+    # caches, so an iteration takes about four times as long (4.0 measured;
+    # 9.2 when the sums were folded for every tile)
+    import time
+    S = serve
+    srv = S.Server(budget_bytes=9 << 30, max_slots=2)
+
+    def seconds(n, steps):
+        # a step's 8 iterations, after a first step with the set-up
+        i = srv.submit(S.POISSON2D, n, seed=1, tol=1e-300, max_iters=8 * steps)
+        best = 1e9
+        for k in range(steps):
+            t = time.perf_counter()
+            srv.step()
+            best = min(best, time.perf_counter() - t)
+        assert srv.active() == 0
+        srv.release(i)
+        return best
+
+    small, large = (seconds(n, 4) for n in (8192, 16384))
+    srv.close()
+    assert large <= 5.5 * small, (small, large)
