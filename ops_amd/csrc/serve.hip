@@ -1059,14 +1059,15 @@ struct opsmi_server_s {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int iters_per_launch = 8, use_graph = 1, max_slots = 0, grid = 0;
-  size_t budget = 0, in_use = 0, max_tiles = 0;
+  size_t budget = 0, in_use = 0;
+  size_t max_tiles = 0, cap_tiles = 0;  // tiles a full arena can need, tiles the tables hold now
   char *arena_base = nullptr;
   Arena arena;
   SolveDev *d_solves = nullptr;
   SolveStat *d_stat = nullptr;  // two copies of max_slots
   int2 *d_tiles = nullptr;
   int *d_ntiles = nullptr;
-  double *d_part = nullptr, *d_setup_part = nullptr;
+  double *d_part = nullptr;  // kPart planes of cap_tiles; set-up sums too (no iteration leaves any behind)
   SolveStat *h_stat = nullptr;  // pinned
   Staging staging;              // fetched solutions
   std::vector<SolveDev> h_solves;
@@ -1126,12 +1127,46 @@ void launch_iterations(opsmi_server S, hipStream_t st, int iters) {
   const dim3 blk(kWave, kWavesPerBlock);
   for (int k = 0; k < iters; k++) {
     hipLaunchKernelGGL(sk_sweep, dim3(S->grid), blk, 0, st, S->d_solves, S->d_stat, S->d_stat + S->max_slots,
-                       S->d_tiles, S->d_ntiles, S->d_part, S->max_tiles);
+                       S->d_tiles, S->d_ntiles, S->d_part, S->cap_tiles);
     hipLaunchKernelGGL(sk_update, dim3(S->grid), blk, 0, st, S->d_solves, S->d_stat + S->max_slots, S->d_stat,
-                       S->d_tiles, S->d_ntiles, S->d_part, S->max_tiles);
+                       S->d_tiles, S->d_ntiles, S->d_part, S->cap_tiles);
   }
   hipLaunchKernelGGL(sk_finish, dim3(S->max_slots), dim3(256), 0, st, S->d_solves, S->d_stat, S->d_part,
-                     S->max_tiles);
+                     S->cap_tiles);
+}
+
+// Tables (tile list and partial sums) for `need` tiles; false when there is no
+// memory for them.  Sized for every tile the arena could ever hold they would
+// take 0.5 % of the budget beside it (1.2 GB at 200 GB), most of it never used:
+// they start at kFirstTiles and at least double.
+constexpr size_t kFirstTiles = 16384;
+bool have_tables(opsmi_server S, size_t need) {
+  if (need <= S->cap_tiles) return true;
+  OPSMI_HIP(hipStreamSynchronize(S->stream));  // set-up kernels use the sums
+  for (size_t cap : {std::min(S->max_tiles, std::max(need, 2 * S->cap_tiles)), need}) {
+    int2 *tiles = nullptr;
+    double *part = nullptr;
+    hipError_t e = hipMalloc(&tiles, sizeof(int2) * cap);
+    if (e == hipSuccess) e = hipMalloc(&part, sizeof(double) * kPart * cap);
+    if (e == hipSuccess) {
+      (void)hipFree(S->d_tiles);
+      (void)hipFree(S->d_part);
+      S->d_tiles = tiles;
+      S->d_part = part;
+      S->cap_tiles = cap;
+      S->dirty = true;
+      // the captured launches hold the old addresses
+      if (S->exec) OPSMI_HIP(hipGraphExecDestroy(S->exec));
+      if (S->graph) OPSMI_HIP(hipGraphDestroy(S->graph));
+      S->exec = nullptr;
+      S->graph = nullptr;
+      return true;
+    }
+    (void)hipFree(tiles);
+    if (e != hipErrorOutOfMemory) OPSMI_HIP(e);
+    (void)hipGetLastError();
+  }
+  return false;
 }
 
 // admits the queue head while a slot and memory are free; sets up on device
@@ -1155,6 +1190,11 @@ void admit(opsmi_server S) {
     if ((size_t)(S->tiles_active + nt) > S->max_tiles) {
       S->arena.release(off, g.bytes);
       return;
+    }
+    if (!have_tables(S, (size_t)(S->tiles_active + nt))) {
+      S->arena.release(off, g.bytes);
+      if (S->n_active == 0) fail(OPS_RUNTIME_ERROR, "opsmi_serve: no device memory for the tile tables of a solve");
+      return;  // with the tables there are, once the solves before it are done
     }
     S->tiles_active += nt;
     S->queue.pop_front();
@@ -1262,8 +1302,8 @@ void admit(opsmi_server S) {
       hipLaunchKernelGGL(sk_heat_coefs, dim3(gb), dim3(256), 0, st, d);
     }
     hipLaunchKernelGGL(sk_first_residual, dim3((unsigned)nt), dim3(kWave, kWavesPerBlock), 0, st, d, R.q.seed,
-                       S->d_setup_part);
-    hipLaunchKernelGGL(sk_first_fold, dim3(1), dim3(256), 0, st, S->d_stat + slot, (const double *)S->d_setup_part,
+                       S->d_part);
+    hipLaunchKernelGGL(sk_first_fold, dim3(1), dim3(256), 0, st, S->d_stat + slot, (const double *)S->d_part,
                        (int)nt, R.q.tol, R.q.max_iters);
     OPSMI_HIP(hipGetLastError());
     S->dirty = true;
@@ -1346,10 +1386,8 @@ opsmi_server opsmi_serve_create(size_t hbm_budget, int max_slots, int iters_per_
   S->arena.init(S->budget);
   OPSMI_HIP(hipMalloc(&S->d_solves, sizeof(SolveDev) * max_slots));
   OPSMI_HIP(hipMalloc(&S->d_stat, 2 * sizeof(SolveStat) * max_slots));
-  OPSMI_HIP(hipMalloc(&S->d_tiles, sizeof(int2) * S->max_tiles));
   OPSMI_HIP(hipMalloc(&S->d_ntiles, sizeof(int)));
-  OPSMI_HIP(hipMalloc(&S->d_part, sizeof(double) * kPart * S->max_tiles));
-  OPSMI_HIP(hipMalloc(&S->d_setup_part, sizeof(double) * S->max_tiles));
+  if (!have_tables(S, std::min(S->max_tiles, kFirstTiles))) OPSMI_HIP(hipErrorOutOfMemory);
   OPSMI_HIP(hipHostMalloc((void **)&S->h_stat, sizeof(SolveStat) * max_slots, hipHostMallocDefault));
   OPSMI_HIP(hipMemsetAsync(S->d_stat, 0, 2 * sizeof(SolveStat) * max_slots, S->stream));
   S->h_solves.assign(max_slots, SolveDev{});
@@ -1567,7 +1605,6 @@ void opsmi_serve_destroy(opsmi_server S) {
   (void)hipFree(S->d_tiles);
   (void)hipFree(S->d_ntiles);
   (void)hipFree(S->d_part);
-  (void)hipFree(S->d_setup_part);
   (void)hipHostFree(S->h_stat);
   S->staging.release();
   if (S->stream) (void)hipStreamDestroy(S->stream);

@@ -335,3 +335,62 @@ def test_iteration_time_grows_with_the_points(serve):
     small, large = (seconds(n, 4) for n in (8192, 16384))
     srv.close()
     assert large <= 5.5 * small, (small, large)
+
+
+def test_tables_beside_the_budget_stay_small(serve):
+    # a server takes its budget and little more (0.6 % of it, 400 MB here, when
+    # the tables were sized for every tile the budget could hold; the runtime
+    # reports large allocations 0.2 % smaller than they were asked for)
+    import ctypes
+    from ops_amd import ops
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert ops.lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    budget = 64 << 30
+    free = free_bytes()
+    srv = serve.Server(budget_bytes=budget, max_slots=64)
+    taken = free - free_bytes()
+    srv.close()
+    assert taken <= budget + (32 << 20), taken - budget
+
+
+def test_tables_grow_while_solves_run(serve):
+    # tables start at 16384 tiles: a solve of 71 x 563 tiles and one of 40 x 313
+    # join while another is under way; the same bits as alone
+    S = serve
+    reqs = [(300, 400), (9000, 6), (5000, 9), (200, 50)]
+    srv = S.Server(budget_bytes=5 << 30, max_slots=8, iters_per_launch=4)
+    ids = [srv.submit(S.POISSON2D, reqs[0][0], seed=70, tol=1e-300, max_iters=reqs[0][1])]
+    srv.step()
+    assert srv.active() == 1
+    ids += [srv.submit(S.POISSON2D, n, seed=70, tol=1e-300, max_iters=m) for n, m in reqs[1:]]
+    out = srv.run()
+    srv.close()
+    for i, (n, m) in zip(ids, reqs):
+        alone = S.Server(budget_bytes=5 << 30, max_slots=2, iters_per_launch=4)
+        j = alone.submit(S.POISSON2D, n, seed=70, tol=1e-300, max_iters=m)
+        d, x = alone.run()[j]
+        alone.close()
+        assert d["iters"] == out[i][0]["iters"] == m and d["rr"] == out[i][0]["rr"]
+        assert np.array_equal(x, out[i][1]), n
+
+
+def test_tables_hold_a_full_arena(serve):
+    # the most tiles for the memory: sides one point past a tile's width, 66
+    # tiles each, in an arena that holds sixteen of them and no more; each with
+    # its own sums (four planes of them)
+    S = serve
+    n = 129
+    srv = S.Server(budget_bytes=16 * S.request_bytes(S.POISSON2D, n), max_slots=17)
+    ids = [srv.submit(S.POISSON2D, n, seed=80 + k) for k in range(17)]
+    srv.step()
+    assert srv.active() == 16 and srv.queued() == 1
+    out = srv.run()
+    srv.close()
+    for k, i in enumerate(ids):
+        d, x = _run_alone(S, S.POISSON2D, n, 80 + k)
+        assert d["iters"] == out[i][0]["iters"] and d["rr"] == out[i][0]["rr"]
+        assert np.array_equal(x, out[i][1]), k
