@@ -92,3 +92,10 @@ def test_declaration_with_data_and_no_points(gpu_ops, size):
     blk = ops.ops_decl_block(nd, "empty")
     d = ops.ops_decl_dat(blk, size, [0] * nd, [0] * nd, data=np.zeros(size[::-1]), name="d")
     ops.ops_free_dat(d)
+
+
+@pytest.mark.parametrize("size,halo", [([256], 1), ([257], 1), ([3], 1), ([65536, 3], 1), ([65537, 3], 1),
+                                       ([70000, 2, 2], 1), ([200000], 2)])
+def test_boxes_on_both_sides_of_the_copy_rules(gpu_ops, size, halo):
+    """rows around the widths (2 KiB single, 512 KiB) that go by a copy call"""
+    test_boxes_equal_numpy_slices(gpu_ops, size, halo, 1, False, np.float64)
