@@ -410,11 +410,8 @@ __global__ __launch_bounds__(64) void k_thomas_x(const T *__restrict__ a, const 
 // reciprocals (same quotients by Markstein's correction) saved nothing after
 // its range checks.  Microseconds along x / y / z, before and now: 256^3
 // 346 / 775 / 900 and 354 / 405 / 365, 200 x 130 x 97 63 / 118 / 148 and
-// 65 / 60 / 52.  Two rows a thread; 4 and 8 rows took 387 / 403 / 389 and
-// 384 / 417 / 388 at 256^3, so longer systems only, which would otherwise
-// leave a workgroup one system, take 4.  The operations of a row are the
+// 65 / 60 / 52.  Two rows a thread (pcr_rows).  The operations of a row are the
 // algorithm's, in its order.
-constexpr int kPcrShort = 256;  // rows up to which a thread takes two
 
 template <class T>
 struct PcrRow {
@@ -499,7 +496,11 @@ __global__ __launch_bounds__(512) void k_pcr(const T *__restrict__ a, const T *_
     for (int k = 0; k < ROWS; k++) {
       const bool lo = k >= m, hi = k + m < ROWS && j + (k + m) * J < n;
       const int l = k >= m ? k - m : k, h = k + m < ROWS ? k + m : k;
-      x[k] = pcr_step(r[k], lo, r[l], hi, r[h]);
+      x[k] = r[k];
+      // along x a wave without rows here, or whose rows have no neighbour left,
+      // skips the divisions (257 rows 78 -> 76 us); across systems every wave
+      // has some (256 rows 56 us, 58 with the condition)
+      if (!ALONG || (j + k * J < n && (lo || hi))) x[k] = pcr_step(r[k], lo, r[l], hi, r[h]);
     }
 #pragma unroll
     for (int k = 0; k < ROWS; k++) r[k] = x[k];
@@ -516,15 +517,23 @@ __global__ __launch_bounds__(512) void k_pcr(const T *__restrict__ a, const T *_
   }
 }
 
+// rows a thread holds.  4 and 8 took 387 / 403 / 389 and 384 / 417 / 388 us
+// along x / y / z at 256^3 in FP64, 2 354 / 405 / 365.  Longer systems across
+// y and z, of which a workgroup would have one or two, take 4; along x they
+// take 2 all the same (3e6 points in FP64, one workgroup per system first, then
+// 4 rows and 2: 257 rows 74, 81 and 76 us, 400 rows 70, 76 and 69, 512 rows 61,
+// 68 and 60, 1024 rows 76, 74 and 65; in FP32 512 rows 45, 37 and 35).
+inline int pcr_rows(int n, bool along) { return along || n <= 256 ? 2 : 4; }
+
 // threads per system and systems per workgroup
 struct PcrShape {
   int S, J;
   size_t lds;
 };
-inline PcrShape pcr_shape(int n, size_t es) {
+inline PcrShape pcr_shape(int n, size_t es, int rows) {
   PcrShape p;
   p.J = 1;
-  while (p.J * (n <= kPcrShort ? 2 : 4) < n) p.J *= 2;
+  while (p.J * rows < n) p.J *= 2;
   // 128 bytes of systems where their rows then fit the 64 KiB of LDS a
   // workgroup may ask for, at most 512 threads; fewer systems for long ones
   p.S = (int)(128 / es);
@@ -655,7 +664,8 @@ void trid_run(int ndim, int solvedim, int *range, ops_dat a, ops_dat b, ops_dat 
   bool pcr = ctx && ctx->strategy == 3;
   if (pcr) {
     if (g.n > 1024) fail(OPS_NOT_IMPLEMENTED, "Tridsolver error: PCR supports systems of at most 1024 rows");
-    const PcrShape ps = pcr_shape((int)g.n, es);
+    const int per = pcr_rows((int)g.n, solvedim == 0);
+    const PcrShape ps = pcr_shape((int)g.n, es, per);
     const unsigned nb = (unsigned)((g.count + ps.S - 1) / ps.S);
     const dim3 block((unsigned)(ps.S * ps.J));
     launch([&](hipStream_t s) {
@@ -672,7 +682,7 @@ void trid_run(int ndim, int solvedim, int *range, ops_dat a, ops_dat b, ops_dat 
         else go(x ? k_pcr<T, false, true, ROWS> : k_pcr<T, false, false, ROWS>, t);
       };
       auto type = [&](auto *t) {
-        if (g.n <= kPcrShort) rows(std::integral_constant<int, 2>{}, t);
+        if (per == 2) rows(std::integral_constant<int, 2>{}, t);
         else rows(std::integral_constant<int, 4>{}, t);
       };
       if (dt == DT_F64) type((double *)nullptr);

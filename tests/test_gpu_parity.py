@@ -801,6 +801,15 @@ def test_pcr_shapes_bit_exact(gpu_ops, dtype, n):
         ops.ops_free_dat(q)
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [(255, 3, 2), (258, 5, 1), (383, 2, 3), (511, 3, 2), (514, 2, 2), (767, 3, 1),
+                               (1023, 2, 2)])
+def test_pcr_long_rows_along_x_bit_exact(gpu_ops, dtype, n):
+    """two rows a thread up to 512 threads a system, with and without whole
+    waves of second rows"""
+    test_pcr_shapes_bit_exact(gpu_ops, dtype, n)
+
+
 @pytest.mark.parametrize("n", [(2, 3, 4), (65, 9, 8), (129, 6, 5), (256, 10, 3), (300, 7, 6)])
 def test_preproc_edges_and_remainders(gpu_ops, n):
     """two points per lane: odd lengths, lengths around a wave's 128 points,
