@@ -705,11 +705,12 @@ void trid_run(int ndim, int solvedim, int *range, ops_dat a, ops_dat b, ops_dat 
       for (char *p : {pa, pb, pc, pd, pu})
         if (p && (uintptr_t)p % 16 != 0) v16 = false;
       // half-filled waves (32 systems) while each of those finds a SIMD of its
-      // own: 30 450 systems of 301 in FP64 take 147 us instead of 201, in FP32
-      // 123 instead of 143, 10 000 of 100 40 instead of 43.  Past that the
-      // fuller waves win: 40 000 systems of 301 in FP64 180 us against 238,
-      // 65 536 of 256 217 against 261
-      const bool half = g.count <= 128L * inst().num_cus;
+      // own, in FP32, whose rows are half as long, up to a quarter more.  FP64,
+      // 32 and 64 systems a wave: 30 450 systems of 301 147 and 201 us, 32 000
+      // of 256 111 and 113, 40 000 of 301 238 and 180, 65 536 of 256 261 and
+      // 217.  FP32: 30 450 of 301 123 and 143, 33 124 of 300 138 and 158,
+      // 40 000 134 and 138, 42 000 152 and 143, 65 536 193 and 183
+      const bool half = g.count <= (dt == DT_F32 ? 160L : 128L) * inst().num_cus;
       const int nw = (int)((g.count + (half ? 31 : 63)) / (half ? 32 : 64));
       launch([&](hipStream_t s) {
         auto go = [&](auto v, auto ns, auto *t) {

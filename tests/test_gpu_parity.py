@@ -745,6 +745,12 @@ def test_set_zero_ranges(gpu_ops, dtype, n, lo, hi):
     ops.ops_free_dat(a)
 
 
+@pytest.mark.parametrize("n", [(17, 256, 160), (20, 257, 160)])
+def test_thomas_fp32_wave_shapes_bit_exact(gpu_ops, n):
+    """system counts on both sides of the FP32 switch along x (160 per CU)"""
+    test_thomas_workgroup_shapes_bit_exact(gpu_ops, np.float32, n, 0, 0)
+
+
 def _pcr_numpy(a, b, c, d):
     """parallel cyclic reduction along the last axis in the arrays' own type,
     with the operations and order of the kernel and the oracle"""
