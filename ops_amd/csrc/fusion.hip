@@ -315,10 +315,12 @@ int pois_chain_rule_level2(std::vector<LoopRec> &run, size_t at, hipStream_t s) 
 // kJacWaves waves, and to single rows below kJacFew.  Timed with events:
 // 96 x 70 13.2 us with 16 rows (5 waves), 5.9 us with one; 1500^2 20.9 with 16,
 // 14.1 with 4; at 2048^2 16 rows 18.3-19.1 us, 8 rows 19.1, 4 rows 18.8, 2 rows
-// 18.2, 1 row 25.2.  A is stored past the caches: the next pass reads it at
+// 18.2, 1 row 25.2.  20 iterations, 8 rows and 16: 4094 x 1100 (2208 waves of
+// 16 rows) 739 and 759 us, 2300^2 (2592) 802 and 783, 2800^2 (3850) 1004 and
+// 976, 4094 x 2000 (4000) 1065 and 1038.  A is stored past the caches: the next pass reads it at
 // the halo only, and Anew, which it reads throughout, keeps the room (4094^2
 // 89 us with plain stores, 70 us so; Anew stored so too: 86 us).
-constexpr int kJacRows = 16, kJacWaves = 4096, kJacFew = 1024;
+constexpr int kJacRows = 16, kJacWaves = 2560, kJacFew = 1024;
 
 template <class T>
 struct JacPtrs {
