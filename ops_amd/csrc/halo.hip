@@ -113,12 +113,15 @@ struct CopyHalo {
   unsigned ext0, ext1, n;  // buffer extents 0 and 1, values in total
   int dim;
 };
-// 36 descriptors stay within a launch's 4 KiB of arguments, so nothing is
-// uploaded and a call keeps no table: pointers are the dats' at this call
+// Descriptors travel as kernel arguments, so nothing is uploaded and a call
+// keeps no table: pointers are the dats' at this call.  36 of 96 bytes, 3.4 KiB
+// of the 4 a launch takes, leave room for the runtime's own arguments (some
+// 256 bytes); a larger group takes another launch, 2.5 us.
 constexpr int kHalosPerLaunch = 36;
 struct CopyHalos {
   CopyHalo h[kHalosPerLaunch];
 };
+static_assert(sizeof(CopyHalos) + 256 <= 4096, "kernel arguments of a halo launch");
 
 // Bounded by launches and latency, not bytes: twelve 250 x 181 blocks with
 // two-point halos (0.2 MB in 34 halos) took 271 us in 68 launches, 6 us in

@@ -160,13 +160,6 @@ __device__ __forceinline__ void store_partial(double v, double *dst, double (*sh
   block_reduce<double, OPS_INC, 1>(acc, sh);
   if (threadIdx.x == 0 && threadIdx.y == 0) *dst = acc[0];
 }
-template <int D>
-__device__ __forceinline__ void store_partials(double (&acc)[D], double *dst, double (*sh)[D]) {
-  block_reduce<double, OPS_INC, D>(acc, sh);
-  if (threadIdx.x == 0 && threadIdx.y == 0)
-#pragma unroll
-    for (int q = 0; q < D; q++) dst[q] = acc[q];
-}
 
 __device__ __forceinline__ Ptr<float> PF32(float *a, const SolveDev &d) { return Ptr<float>{a, d.sy32, d.sz32}; }
 __device__ __forceinline__ Ptr<const float> PF32C(const float *a, const SolveDev &d) {
