@@ -311,16 +311,16 @@ int pois_chain_rule_level2(std::vector<LoopRec> &run, size_t at, hipStream_t s) 
 // lanes (shuffles) and, at the strip ends, one scalar load.
 //
 // Bounded by HBM on large grids and by the march's latency (0.6 us a row) on
-// small ones: kJacRows rows a wave, halved while the grid has fewer than
-// kJacWaves waves, and to single rows below kJacFew.  Timed with events:
-// 96 x 70 13.2 us with 16 rows (5 waves), 5.9 us with one; 1500^2 20.9 with 16,
-// 14.1 with 4; at 2048^2 16 rows 18.3-19.1 us, 8 rows 19.1, 4 rows 18.8, 2 rows
-// 18.2, 1 row 25.2.  20 iterations, 8 rows and 16: 4094 x 1100 (2208 waves of
-// 16 rows) 739 and 759 us, 2300^2 (2592) 802 and 783, 2800^2 (3850) 1004 and
-// 976, 4094 x 2000 (4000) 1065 and 1038.  A is stored past the caches: the next pass reads it at
-// the halo only, and Anew, which it reads throughout, keeps the room (4094^2
-// 89 us with plain stores, 70 us so; Anew stored so too: 86 us).
-constexpr int kJacRows = 16, kJacWaves = 2560, kJacFew = 1024;
+// small ones: kJacRows rows a wave where that leaves kJacLong waves (ten a CU),
+// else the most of 8, 4 and 2 that leaves more than kJacWaves, and single rows
+// below kJacFew.  Microseconds per iteration of the application with 16 / 8 / 4 /
+// 2 rows (16 with plain stores, loads under conditions): 600^2 19.5 / 14.9 /
+// 12.7 / 12.0 (19.9), 1500^2 22.8 / 18.5 / 17.6 / 17.8 (23.8), 2048^2 22.4 / 23.2
+// / 22.5 / 23.1 (22.9), 4094 x 1100 26.6 / 25.3 / 26.2 / 26.4 (27.1), 2800^2 33.4
+// / 34.9 / 34.7 / 36.0 (33.9), 4094 x 2000 35.2 / 38.1 / 36.6 / 37.9 (35.4).  A is stored past the caches: the next pass reads it at the halo only,
+// and Anew, which it reads throughout, keeps the room (4094^2 89 us with plain
+// stores, 70 us so; Anew stored so too: 86 us).
+constexpr int kJacRows = 16, kJacLong = 2560, kJacWaves = 4096, kJacFew = 1024;
 
 template <class T>
 struct JacPtrs {
@@ -405,7 +405,9 @@ void launch_jacobi_chain(const LoopRec &cp, const LoopRec &jac, const Range3 &R)
   const long nx = R.x1 - R.x0, ny = R.y1 - R.y0;
   const unsigned gx = (unsigned)((nx + kWave * V - 1) / (kWave * V));
   int rows = kJacRows;
-  while (rows > 1 && gx * ((ny + rows - 1) / rows) < (rows > 2 ? kJacWaves : kJacFew)) rows /= 2;
+  while (rows > 1 &&
+         gx * ((ny + rows - 1) / rows) < (rows == kJacRows ? kJacLong : rows > 2 ? kJacWaves + 1 : kJacFew))
+    rows /= 2;
   const unsigned gy = (unsigned)((ny + kWavesPerBlock * rows - 1) / (kWavesPerBlock * rows));
   ensure_partials((size_t)gx * gy * sizeof(T));
   JacPtrs<T> c;
