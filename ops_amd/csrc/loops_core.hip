@@ -422,7 +422,7 @@ LoopRec make_poisson3_loop(const char *name, const ops_arg *args, int nargs, con
 // apps/c/adi/preproc_kernel.h:4-39.  Bounded by its stores (10 arrays out, 1
 // in, 88 bytes a point): two points per lane and, beyond the Infinity Cache,
 // non-temporal 16-byte stores.  256^3: 368 us (4.0 TB/s) with one point per
-// lane, 325 us (4.5 TB/s) now.
+// lane, 325 to 337 us (4.4 to 4.5 TB/s) now.
 struct Preproc {
   OPSMI_NO_RED
   static constexpr int kVec = 2;

@@ -46,12 +46,17 @@ namespace {
 // Default tile parameter per size class (size_class): rows per wave of a 2D
 // tile, z planes of a 3D tile.  A tile is worked through serially, so small
 // solves take short tiles (more workgroups) and large ones long tiles (fewer
-// rim re-reads).  Microseconds per CG iteration of one solve alone:
-//   2D side    1 row   2 rows  4 rows   |  3D side   4      8      16 planes
-//     256       17.9    18.6    20.2    |    32     23.5   30.0   42.3
-//     512       20.1    19.6    21.0    |    64     24.7   29.8   41.0
-//    1000       35.7    29.4    28.0    |    96     42.4   41.2   51.4
-//    2000      104.9    85.6    76.5    |   200    242.4  261.1  197.5
+// rim re-reads).  Microseconds per CG iteration of one FP64 solve alone:
+//   2D side   1 row   2 rows  4 rows  8 rows |  3D side  4      8      16     32 planes
+//     128      12.6    13.8    15.8    19.3  |    32    16.5   21.9   32.2   53.4
+//     256      12.5    13.6    15.8    20.0  |    64    17.8   22.1   33.5   54.4
+//     512      14.3    14.7    16.6    20.5  |    96    27.4   31.3   38.3   60.3
+//     700      20.0    17.4    19.1    23.2  |   128    45.8   45.5   47.2   64.2
+//    1000      28.7    24.2    22.0    24.6  |   200   226    260    213    221
+//    2000      85      71      63      64    |   256   427    401    386    391
+//    4096     377     324     309     302    |   512  3059   3009   2995   2987
+// A class's value is within 10 % of its sides' best; opsmi_serve_autotune
+// measures on the card at hand.
 constexpr int kRows2D[3] = {1, 2, 4};
 constexpr int kChunk3D[3] = {4, 4, 16};
 constexpr int kPart = 4;  // partial sums per tile: planes 0-2 of the update, plane 3 p.w
@@ -589,9 +594,19 @@ __device__ __forceinline__ void correct_tile(const SolveDev &d, const TileBox &b
 // 5.2 us a launch at 64^2), bandwidth-bound on large ones.  A tile's first
 // loads are issued before its solve's sums are folded.  Microseconds per CG
 // iteration of one solve alone, five launches and now:
-//   2D 64^2 17.8 and 12.5, 512^2 19.6 and 14.7, 1000^2 28.0 and 24.0,
-//   2000^2 76.5 and 63.7 (5.0 TB/s of 80 bytes a point); 3D 64^3 24.7 and
-//   17.9, 128^3 60.8 and 47.8; FP32-inner 2D 1000^2 25.0 and 19.4
+//   2D 64^2 17.8 and 12.3, 512^2 19.6 and 14.7, 1000^2 28.0 and 24.0, 2000^2
+//   76.5 and 63 (5.1 TB/s of 80 bytes a point), 4096^2 335 and 309, 8192^2
+//   1392 and 1188; FP32-inner 1000^2 25.0 and 19.3, 8192^2 721 and 634
+//   3D 64^3 24.7 and 17.7, 128^3 60.8 and 47.2, 200^3 245 and 214, 300^3 719
+//   and 724, 512^3 2995 and 3002; FP32-inner 200^3 278 and 121, 384^3 769 and 772
+// Between them 3D solves whose fields straddle the Infinity Cache lose: 240^3
+// 313 and 330, 256^3 365 and 386, FP32-inner 256^3 196 and 210.  The sweep
+// there takes 223 us for 48 bytes a point (3.6 TB/s; the update 165, 5.7): it
+// fetches 1.23 times its arrays, the five launches' LDS column 1.14 times.
+// Tried there: neighbours along x by lane shuffles and uniform row addresses,
+// 382 at 256^3 (FP32-inner 202); with the coefficients loaded past the caches
+// 390 (189), 5 % slower at 128^3; tiles of 64 planes 374, 20 % slower at 200^3;
+// four waves a SIMD, which spill, 524.
 __global__ __launch_bounds__(256) void sk_sweep(const SolveDev *__restrict__ S, const SolveStat *__restrict__ in,
                                                 SolveStat *__restrict__ out, const int2 *__restrict__ tiles,
                                                 const int *__restrict__ ntiles, double *part, size_t np) {

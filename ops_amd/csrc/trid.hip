@@ -408,9 +408,9 @@ __global__ __launch_bounds__(64) void k_thomas_x(const T *__restrict__ a, const 
 // of every 128-byte line along y and z).  Bounded by vector arithmetic, 62
 // instructions a row and step, two divisions among them: sharing their
 // reciprocals (same quotients by Markstein's correction) saved nothing after
-// its range checks.  Microseconds along x / y / z, before and now: 256^3
-// 346 / 775 / 900 and 354 / 405 / 365, 200 x 130 x 97 63 / 118 / 148 and
-// 65 / 60 / 52.  Two rows a thread (pcr_rows).  The operations of a row are the
+// its range checks.  Microseconds along x / y / z, one workgroup per system and
+// now: 256^3 366 / 774 / 887 and 323 / 317 / 310, 200 x 130 x 97 63 / 118 / 148
+// and 64 / 61 / 53.  Two rows a thread (pcr_rows).  The operations of a row are the
 // algorithm's, in its order.
 
 template <class T>
@@ -517,12 +517,13 @@ __global__ __launch_bounds__(512) void k_pcr(const T *__restrict__ a, const T *_
   }
 }
 
-// rows a thread holds.  4 and 8 took 387 / 403 / 389 and 384 / 417 / 388 us
-// along x / y / z at 256^3 in FP64, 2 354 / 405 / 365.  Longer systems across
-// y and z, of which a workgroup would have one or two, take 4; along x they
-// take 2 all the same (3e6 points in FP64, one workgroup per system first, then
-// 4 rows and 2: 257 rows 74, 81 and 76 us, 400 rows 70, 76 and 69, 512 rows 61,
-// 68 and 60, 1024 rows 76, 74 and 65; in FP32 512 rows 45, 37 and 35).
+// rows a thread holds.  4 took 368 / 333 / 321 us along x / y / z at 256^3 in
+// FP64, 2 323 / 317 / 310, and 71 / 61 / 53 and 64 / 61 / 53 at 200 x 130 x 97.
+// Longer systems across y and z, of which a workgroup would have one or two,
+// take 4; along x they take 2 all the same (3e6 points in FP64, one workgroup
+// per system first, then 4 rows and 2: 257 rows 74, 81 and 76 us, 400 rows 70,
+// 76 and 69, 512 rows 61, 68 and 60, 1024 rows 76, 74 and 65; in FP32 512 rows
+// 45, 37 and 35).
 inline int pcr_rows(int n, bool along) { return along || n <= 256 ? 2 : 4; }
 
 // threads per system and systems per workgroup

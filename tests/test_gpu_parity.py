@@ -698,8 +698,8 @@ def test_stencil27_column_bit_exact(gpu_ops, n):
     ((48, 33, 3), 0, 0), ((35, 31, 2), 0, 0), ((40, 13, 5), 4, 1), ((40, 13, 5), 1, 2), ((1, 7, 3), 0, 0)])
 def test_thomas_workgroup_shapes_bit_exact(gpu_ops, dtype, n, lo, hi):
     """system counts on both sides of the switches between workgroup shapes
-    (128 systems per CU along x, 64 along y and z, at 256 CUs) and of whole
-    waves; lengths around a chunk of 16; ranges that start on and off 16 bytes"""
+    (in FP64 128 systems per CU along x, in both types 64 along y and z, at
+    256 CUs) and of whole waves; lengths around a chunk of 16; ranges that start on and off 16 bytes"""
     ops = gpu_ops
     rng = np.random.RandomState(6)
     shape = n[::-1]
