@@ -1012,6 +1012,9 @@ ops_dat ops_decl_dat_char(ops_block block, int dim, int *dsize, int *base, int *
       if (on_device) OPSMI_HIP(hipMemcpy2D(b.base, b.pitch, from, upitch, upitch, rows, hipMemcpyDefault));
       else box_copy(I.staging, I.stream, b, from, true);
     }
+    // the copy call may return before a device buffer has been copied, and the
+    // library's stream does not wait for the default one
+    if (on_device) OPSMI_HIP(hipStreamSynchronize(nullptr));
   }
   d->data = nullptr;
   d->user_managed = 0;

@@ -99,3 +99,27 @@ def test_declaration_with_data_and_no_points(gpu_ops, size):
 def test_boxes_on_both_sides_of_the_copy_rules(gpu_ops, size, halo):
     """rows around the widths (2 KiB single, 512 KiB) that go by a copy call"""
     test_boxes_equal_numpy_slices(gpu_ops, size, halo, 1, False, np.float64)
+
+
+def test_declaration_with_data_in_device_memory(gpu_ops):
+    """the data pointer may be device memory (here another dat's, rows without
+    padding, 512 MiB): copied when the call returns, whichever stream the
+    library works on"""
+    import ctypes as C
+    ops = gpu_ops
+    nx, ny = 4094, 16382
+    blk = ops.ops_decl_block(2, "ondevice")
+    a = ops.ops_decl_dat(blk, [nx, ny], name="a")
+    for y in (0, 1, ny // 2, ny - 1):
+        ops.ops_dat_set_data_slab(a, [0, nx, y, y + 1], np.arange(nx, dtype=np.float64).reshape(1, nx) + 1000.5 * y)
+    space = C.c_int(ops.OPS_DEVICE)
+    addr = ops._call("ops_dat_get_raw_pointer", a.ptr, 0, None, C.byref(space)) - 8 * (1 + (nx + 2))  # point (-1, -1)
+    p = ops._call("ops_decl_dat_char", blk.ptr, 1, ops._ints([nx, ny]), ops._ints([0, 0]), ops._ints([-1, -1]),
+                  ops._ints([1, 1]), ops._ints([1, 1]), addr, 8, b"double", b"b")
+    b = ops.Dat(p, blk, [nx, ny], [-1, -1], [1, 1], np.dtype(np.float64), "b", 1)
+    last = ops.ops_dat_fetch_data_slab(b, [0, nx, ny - 1, ny])
+    ops._call("ops_dat_release_raw_data", a.ptr, 0, ops.OPS_READ)
+    assert np.array_equal(last, ops.ops_dat_fetch_data_slab(a, [0, nx, ny - 1, ny])) and last[0, 1] != 0
+    assert np.array_equal(ops.get_whole(b), ops.get_whole(a))
+    ops.ops_free_dat(a)
+    ops.ops_free_dat(b)
